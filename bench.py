@@ -65,7 +65,7 @@ def kernel_bytes(cls: str, npl: int, nk: int, nb: int, n_e: int, solver: str = "
     return {"grad_col": 2 * s, "grad_row": (4 if (coulomb and hf_fused) else 3) * s, "grad_fused": 2 * s, "kgrad": 2 * s, "comm": comm * s,
             "hf_row": 2 * s,
             "hf_col": 2.5 * s, "peierls_col": (2 + n_e) * s,
-            "peierls_row": 2 * s}.get(cls, 0.0)
+            "peierls_row": 2 * s, "hf_plane": 3.5 * s, "peierls_plane": (2 + n_e) * s}.get(cls, 0.0)
 
 
 def cpu_baseline(params: dict, steps: int, integ: str, bytes_per_kstep: float = 0.0, budget_s: float = 18.0):
@@ -250,8 +250,8 @@ def main():
     sim.steps(args.steps)
     eng.synchronize()
     elapsed_direct = time.perf_counter() - t1
-    classes = ["grad_col", "grad_row", "grad_fused", "kgrad", "comm", "hf_row", "hf_col", "peierls_col",
-               "peierls_row"]
+    classes = ["grad_col", "grad_row", "grad_fused", "kgrad", "comm", "hf_row", "hf_col", "hf_plane", "peierls_col",
+               "peierls_row", "peierls_plane"]
     times = {c: eng.timing_get(c) for c in classes}
     eng.timing_enable(False)
 

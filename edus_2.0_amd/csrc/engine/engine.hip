@@ -232,6 +232,7 @@ Engine::Engine(const edus_desc& d, const EngineOptions& opt)
         HIP_CHECK(hipMemcpyAsync(kst_dev, kst.data(), kst.size() * sizeof(KStencilPoint), hipMemcpyHostToDevice, s));
         HIP_CHECK(hipStreamSynchronize(s));
     }
+    plane_ok = plane_available(N0, N1);
     fac[0] = factorize(N0);
     fac[1] = factorize(N1);
     for (int ax = 0; ax < 2; ++ax) {
@@ -266,6 +267,7 @@ Engine::Engine(const edus_desc& d, const EngineOptions& opt)
         alloc(reinterpret_cast<void**>(&W), size_t(npl) * Nk * sizeof(double));
         HIP_CHECK(hipMemcpyAsync(stage, d.W, full, hipMemcpyHostToDevice, s));
         launch_to_planes_real(stage, W, nb, Nk, layout, s);
+        make_plane_W();
         std::vector<double> hr(nb * nb);
         for (int i = 0; i < nb * nb; ++i) hr[i] = d.hartree[2 * i];  // V is real (ModelCoulomb.cpp:168-176)
         alloc(reinterpret_cast<void**>(&hart), nb * nb * sizeof(double));
@@ -287,6 +289,14 @@ Engine::Engine(const edus_desc& d, const EngineOptions& opt)
     make_f32_fields();  // from the final H0
     HIP_CHECK(hipStreamSynchronize(s));
     HIP_CHECK(hipGetLastError());
+}
+
+// W in the order in which the plane kernel meets the frequencies
+void Engine::make_plane_W()
+{
+    if (!plane_ok) return;
+    alloc(reinterpret_cast<void**>(&Wp), size_t(B) * npl * Nk * sizeof(double));
+    launch_plane_permute(W, Wp, B * npl, N0, N1, s);
 }
 
 // FP32 copies of H0 and xi for the mixed-precision commutator, which then
@@ -755,7 +765,9 @@ void Engine::autotune()
     // gives the faster stage (timed with the commutator that consumes D: the
     // one-pass form leaves different data in the caches); they agree to rounding
     grad_fused = false;
-    if (grad_fused_available(N0, N1) && !kgrad) {
+    if (grad_form_choice(N0, N1) && plane_ok && coulomb && !kgrad) {
+        grad_fused = force_grad != 0;  // derivative and exchange term in one launch
+    } else if (grad_form_choice(N0, N1) && !kgrad) {
         const auto gkey = std::make_tuple(N0, N1, B * npl);
         auto git = tuned_grad().find(gkey);
         if (force_grad >= 0) {  // a batch group keeps its members' form (they differ in rounding)
@@ -874,6 +886,15 @@ void Engine::prime_launch_attributes()
         launch_rotate(nb, layout, kCommMfma64, r, s);
         launch_rotate(nb, layout, kCommMfma32, r, s);
     }
+    if (plane_ok) {
+        PlaneArgs a = plane_args(N0, N1);
+        a.phase = peierls ? 1 : 0;
+        launch_plane(a, s);
+        if (peierls && coulomb) {
+            a.phase = 0;
+            launch_plane(a, s);
+        }
+    }
     if (grad_fused_available(N0, N1)) {
         GradFusedArgs g{};
         g.N0 = N0;
@@ -892,6 +913,10 @@ const double2* Engine::gradient(const double2* in, const double c[2], const doub
     use0 = use0 && N0 > 1;
     use1 = use1 && N1 > 1;
     if (!use0 && !use1) return nullptr;
+    if (plane_pass()) {
+        plane_launch(in, true, c, ctab, false);
+        return D;
+    }
     const double* t0 = ctab ? ctab + 0 : nullptr;
     const double* t1 = ctab ? ctab + 1 : nullptr;
     // the row pass also stores the forward row transform of `in` (the
@@ -929,6 +954,30 @@ const double2* Engine::gradient(const double2* in, const double c[2], const doub
     return D;
 }
 
+void Engine::plane_launch(const double2* in, bool deriv, const double c[2], const double* ctab, bool conv)
+{
+    PlaneArgs a = plane_args(N0, N1);
+    a.in = in;
+    a.out[0] = deriv ? D : nullptr;
+    a.out[1] = conv ? T : nullptr;
+    a.P = B * npl;
+    a.tw0 = tw[0];
+    a.tw1 = tw[1];
+    if (deriv)
+        for (int j = 0; j < 2; ++j) a.coef[j] = c[j];
+    a.coef_tab = ctab;
+    a.coef_stride = 2;
+    a.ppi = npl;
+    a.conv = conv ? 1 : 0;
+    a.Wp = Wp;
+    a.conv_scale = -1.0 / double(Nk);
+    a.r0 = hsum;
+    TimedLaunch t;
+    tbegin(conv ? "hf_plane" : "grad_fused", t);
+    launch_plane(a, s);
+    tend(t);
+}
+
 const double2* Engine::kgradient(const double2* in, const double E[3], const double* E_tab)
 {
     TimedLaunch t;
@@ -944,9 +993,26 @@ const double2* Engine::kgradient(const double2* in, const double E[3], const dou
 // term costs no pass of its own.
 void Engine::fock(const double2* in, bool row_done)
 {
+    if (plane_exchange()) {
+        plane_launch(in, false, nullptr, nullptr, true);
+        return;
+    }
     if (!row_done) axis_fft(1, 1, in, nullptr, T, 0.0, 1.0, nullptr, "hf_row");
     axis_fft(0, 3, T, nullptr, T, 0.0, -1.0 / double(Nk), W, "hf_col", nullptr, nullptr, hsum);
     axis_fft(1, 2, T, nullptr, T, 0.0, 1.0, nullptr, "hf_row");
+}
+
+// D = E . grad rho (as gradient) and, with exchange, T of the same input
+const double2* Engine::spectral_terms(const double2* in, const double c[2], const double* ctab, bool use0, bool use1)
+{
+    if (coulomb && plane_exchange() && ((use0 && N0 > 1) || (use1 && N1 > 1))) {  // both from one launch
+        plane_launch(in, true, c, ctab, true);
+        return D;
+    }
+    bool hf_row = false;  // the exchange term's forward row pass done by the gradient
+    const double2* Dp = gradient(in, c, ctab, use0, use1, coulomb && hf_fuse ? T : nullptr, &hf_row);
+    if (coulomb) fock(in, hf_row);
+    return Dp;
 }
 
 void Engine::transform_to_R(const double2* in, double2* out)
@@ -969,11 +1035,13 @@ void Engine::evaluate(const double2* in, const double E[3], const StageUpdate& u
 {
     double cg[2];
     for (int j = 0; j < 2; ++j) cg[j] = (A[0][j] * E[0] + A[1][j] * E[1] + A[2][j] * E[2]) / (j == 0 ? N0 : N1);
-    bool hf_row = false;  // the exchange term's forward row pass done by the gradient
-    const double2* Dp = kgrad ? ((cg[0] != 0.0 || cg[1] != 0.0) ? kgradient(in, E, nullptr) : nullptr)
-                              : gradient(in, cg, nullptr, cg[0] != 0.0, cg[1] != 0.0,
-                                         coulomb && hf_fuse ? T : nullptr, &hf_row);
-    if (coulomb) fock(in, hf_row);
+    const double2* Dp;
+    if (kgrad) {
+        Dp = (cg[0] != 0.0 || cg[1] != 0.0) ? kgradient(in, E, nullptr) : nullptr;
+        if (coulomb) fock(in);
+    } else {
+        Dp = spectral_terms(in, cg, nullptr, cg[0] != 0.0, cg[1] != 0.0);
+    }
     CommArgs c{};
     c.Nk = Nk;
     c.P = npl;
@@ -1140,6 +1208,8 @@ Engine::Engine(const std::vector<const Engine*>& members)
                                      hipMemcpyDeviceToDevice, s));
         }
     }
+    plane_ok = m0.plane_ok;
+    if (coulomb) make_plane_W();
     // upper-triangle fields when every member has them; the group reads them
     // as its members do (same_group keeps members with different choices apart)
     tri_ok = true;
@@ -1175,11 +1245,13 @@ void Engine::evaluate_tab(const double2* in, int ts, int j, const bool use_axis[
 {
     const size_t row = size_t(ts) * 3 + j;
     const double c0[2] = {0.0, 0.0};
-    bool hf_row = false;  // the exchange term's forward row pass done by the gradient
-    const double2* Dp = kgrad ? ((use_axis[0] || use_axis[1]) ? kgradient(in, nullptr, E_dev + row * B * 3) : nullptr)
-                              : gradient(in, c0, coef_dev + row * B * 2, use_axis[0], use_axis[1],
-                                         coulomb && hf_fuse ? T : nullptr, &hf_row);
-    if (coulomb) fock(in, hf_row);
+    const double2* Dp;
+    if (kgrad) {
+        Dp = (use_axis[0] || use_axis[1]) ? kgradient(in, nullptr, E_dev + row * B * 3) : nullptr;
+        if (coulomb) fock(in);
+    } else {
+        Dp = spectral_terms(in, c0, coef_dev + row * B * 2, use_axis[0], use_axis[1]);
+    }
     CommArgs c{};
     c.Nk = Nk;
     c.P = npl;
@@ -1219,6 +1291,26 @@ void Engine::peierls_sandwich(const double2* in, const double2* const add[3], co
 {
     double th[2];
     for (int j = 0; j < 2; ++j) th[j] = sign * (Av[0] * A[0][j] + Av[1] * A[1][j] + Av[2] * A[2][j]);
+    if (plane_pass()) {
+        PlaneArgs a = plane_args(N0, N1);
+        a.in = in;
+        a.out[0] = out;
+        a.P = B * npl;
+        a.tw0 = tw[0];
+        a.tw1 = tw[1];
+        a.phase = 1;
+        for (int j = 0; j < 2; ++j) a.coef[j] = th[j];
+        for (int d = 0; d < 3; ++d) {  // a zero field component reads nothing
+            const bool use = add && add[d] && addc && addc[d] != 0.0;
+            a.in_add[d] = use ? add[d] : nullptr;
+            a.in_add_c[d] = use ? addc[d] : 0.0;
+        }
+        TimedLaunch t;
+        tbegin("peierls_plane", t);
+        launch_plane(a, s);
+        tend(t);
+        return;
+    }
     const double2* src = in;
     const bool two = N0 > 1 && N1 > 1;
     // the phase of each frequency once per sandwich, not once per element
@@ -1733,7 +1825,7 @@ int edus_set_tuning(edus_ctx* ctx, const edus_tuning* in)
         for (int t : {in->comm_tile, in->comm_tile_ab})
             if (t != 0 && (t < 1 || t > 2 || in->comm_kind == edus::kCommScalar))
                 throw EngineError(EDUS_ERR_ARG, "comm_tile and comm_tile_ab must be 0, or 1 or 2 for the MFMA engines");
-        if (in->grad_fused != 0 && (in->grad_fused != 1 || !edus::grad_fused_available(e.N0, e.N1) || e.kgrad))
+        if (in->grad_fused != 0 && (in->grad_fused != 1 || !edus::grad_form_choice(e.N0, e.N1) || e.kgrad))
             throw EngineError(EDUS_ERR_ARG, "grad_fused must be 0, or 1 on the grids with a one-pass gradient kernel");
         if (in->tri_fields != 0 && (in->tri_fields != 1 || !e.tri_ok))
             throw EngineError(EDUS_ERR_ARG, "tri_fields must be 0, or 1 where H0 and r are Hermitian (FULL layout, "

@@ -110,6 +110,25 @@ class Engine {
     void prime_launch_attributes();
     double2 *U = nullptr, *T = nullptr, *stage = nullptr;
     double *W = nullptr, *hart = nullptr;
+    // the grid's planes fit in LDS (plane_fft.hip); W in that kernel's order
+    bool plane_ok = false;
+    double* Wp = nullptr;
+    void make_plane_W();
+    // Derivative and Peierls phase one work-group per plane: on a grid with a
+    // choice, when the tuning has it (grad_fused); otherwise where an axis would
+    // take the Stockham kernel (45 x 63, 21 planes: 10 us instead of 27; with two
+    // two-step axes the passes are as fast: 60 x 60, 64 planes, 9.7 against 11).
+    // The rule may not depend on the number of stacked instances: a batch
+    // member ends bit for bit where it ends alone.
+    bool plane_pass() const
+    {
+        if (!plane_ok) return false;
+        if (grad_form_choice(N0, N1)) return grad_fused && plane_form(N0, N1);
+        return !fft_choice[0].two_step || !fft_choice[1].two_step;
+    }
+    // with exchange one launch instead of up to five (90 x 90, 64 planes: 19 us
+    // instead of 32)
+    bool plane_exchange() const { return plane_ok && (kgrad || !grad_form_choice(N0, N1) || grad_fused); }
     double2 *hdiag = nullptr, *hsum = nullptr;  // hdiag: set-up only
     int force_kind = -1;  // >= 0: the autotuner keeps this commutator engine (batch groups)
     double *obs_partial = nullptr, *obs_out = nullptr;
@@ -119,7 +138,7 @@ class Engine {
     double2* tw[2] = {nullptr, nullptr};
     FFTFactors fac[2];
     FFTChoice fft_choice[2];  // autotuned kernel and tile per grid axis
-    bool grad_fused = false;  // spectral derivative in one pass per plane (grad_fused.hip)
+    bool grad_fused = false;  // spectral passes one work-group per plane (plane_fft.hip, grad_fused.hip)
     int force_grad = -1;      // >= 0: the autotuner keeps this gradient form (batch groups)
     int comm_kind = kCommScalar;     // engine of the RHS commutator (precision-dependent)
     int comm_kind64 = kCommScalar;   // FP64 engine, also used for set-up products
@@ -199,6 +218,9 @@ class Engine {
     // from the row pass (mode 5) where it can; *fwd1_done says whether it did
     const double2* gradient(const double2* in, const double c[2], const double* ctab, bool use0, bool use1,
                             double2* fwd1 = nullptr, bool* fwd1_done = nullptr);
+    // plane kernel: the derivative of in into D (deriv) and the exchange term into T (conv)
+    const double2* spectral_terms(const double2* in, const double c[2], const double* ctab, bool use0, bool use1);
+    void plane_launch(const double2* in, bool deriv, const double c[2], const double* ctab, bool conv);
     void ensure_hist();
     // exchange term of in into T (+ Hartree diagonal); row_done: T already
     // holds the forward row transform of in (from the gradient's row pass)

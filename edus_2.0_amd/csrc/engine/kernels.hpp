@@ -183,6 +183,46 @@ struct GradFusedArgs {
 bool grad_fused_available(int N0, int N1);
 void launch_grad_fused(const GradFusedArgs& a, hipStream_t s);
 
+// Two-dimensional spectral passes of planes that fit in LDS (plane_fft.hip),
+// one work-group per plane and result.  launch_plane: the derivative of every
+// plane into out[0] (null: none), coef = c_j / N_j or per instance from
+// coef_tab[(plane / ppi) * coef_stride + j], and with conv the convolution with
+// conv_scale * W into out[1] (Wp: W in the kernel's order, from
+// launch_plane_permute), each plane's sum over k into r0; with phase (alone)
+// out[0] = F^-1 exp(i (coef0 R0 + coef1 R1)) F (in + sum_d in_add_c[d] in_add[d]).
+struct PlaneArgs {
+    const double2* in;
+    double2* out[2];
+    int P, N0, N1;
+    int RA0, RB0, RA1, RB1;               // line splits (plane_args)
+    float inv_N0, inv_N1, inv_RB0;
+    const double2 *tw0, *tw1;             // exp(-2 pi i j / N_axis)
+    double coef[2];
+    const double* coef_tab;
+    int coef_stride, ppi;
+    int conv;
+    const double* Wp;
+    double conv_scale;
+    double2* r0;
+    int phase;
+    const double2* in_add[3];
+    double in_add_c[3];
+};
+bool plane_available(int N0, int N1);
+// grids on which the tuning chooses between the one-pass derivative
+// (plane_fft.hip, or grad_fused.hip where the plane does not fit) and axis passes
+inline bool grad_form_choice(int N0, int N1)
+{
+    return N0 == N1 && (N0 == 120 || N0 == 96 || N0 == 90 || N0 == 48);
+}
+// of those, the ones whose one-pass derivative is plane_fft.hip's (90 x 90 and
+// 196 planes: 21.1 us, grad_fused.hip took 23.0; 96 x 96: 22.4 and 28.3; at
+// 48 x 48 and 784 planes grad_fused.hip takes 20.1, plane_fft.hip 22.8)
+inline bool plane_form(int N0, int N1) { return N0 == N1 && (N0 == 96 || N0 == 90); }
+PlaneArgs plane_args(int N0, int N1);  // sizes and line splits
+void launch_plane(const PlaneArgs& a, hipStream_t s);
+void launch_plane_permute(const double* W, double* Wp, int P, int N0, int N1, hipStream_t s);
+
 // Gauge rotation per k (Operator::go_to_bloch / go_to_wannier): out =
 // U^dagger in U (to_bloch) or U in U^dagger, in is planes [npl][Nk] of the
 // launch's input layout, U full planes [nb*nb][Nk] (U(a, n) in plane a*nb + n,

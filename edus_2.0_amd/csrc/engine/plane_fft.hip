@@ -1,0 +1,418 @@
+// Two-dimensional spectral passes with a whole plane in LDS.
+//
+// The right-hand side needs, per plane, the derivative
+//   D = F^-1 diag(i (c0 R0 + c1 R1)) F rho
+// (kGradient_definitions.hpp:35-41 inside Functional_SourceTerm.hpp:20-24),
+// with exchange also the convolution T = F^-1[-W o F rho / N]
+// (Coulomb.cpp:134-180), and in the Peierls gauge S_A[H] = F^-1 exp(i A.R) F H
+// (Simulation.cpp:876-899).  Where a plane fits in the LDS of one CU, one
+// work-group does the whole two-dimensional sandwich there: the plane is read
+// once and its result written once, in one launch, where the axis passes
+// (fft_two.hip, fft_axis.hip) take two to five launches with a plane set
+// through memory between each.  With exchange the derivative and the
+// convolution of one plane are two work-groups of the same launch.
+//
+// Every line is n = RA * RB with both factors at most 16, chosen on the host
+// (plane_plan); the factors are run-time values and each step is dispatched on
+// its radix, so that every axis length with such a split shares one kernel.
+// Element j = ja RB + jb, frequency k = ka + RA kb:
+//   A   DFT_RA over ja, times w^(jb ka), to position ka RB + jb;
+//   B   DFT_RB over jb, to position ka RB + kb, which then holds frequency
+//       ka + RA kb; the inverse runs B, then A, back to natural order.
+// Steps work in place on the plane's array in LDS (a task reads and writes its
+// own positions; one barrier between steps).  Axis 0 is outermost: its A step
+// loads from memory and its inverse A step stores, coalesced over columns;
+// the multiplier is applied between B and its inverse of axis 1, in registers.
+// Neighbouring lanes take neighbouring lines: columns are adjacent words, and
+// rows are N1 | 1 elements apart, so neither axis has bank conflicts.
+//
+// What bounds it: the FP64 transforms and LDS round trips (12 of 16 B per
+// element for both axes) of one plane on one CU; with fewer planes than CUs the
+// chip is partly idle, which the saved launches and passes outweigh.  Measured
+// (derivative): 45 x 63, 21 planes 10 us, two Stockham passes 27; 90 x 90 with
+// exchange, 64 planes 18.9 us, four axis passes 32; 96 x 96, 784 planes 82 us
+// (2.8 TB/s), two axis passes 90.  A derivative alone on a small grid with
+// two-step kernels on both axes is left to them (30 x 30: 6.3 against 7.5 us for
+// both axes but 5.1 against 3.5 for one; 60 x 60, 64 planes: 11.2 against 9.7).
+#include <algorithm>
+#include <mutex>
+
+#include "common.hpp"
+#include "fft_reg.hpp"
+#include "kernels.hpp"
+
+namespace edus {
+
+namespace {
+
+using reg::sfor;
+
+constexpr size_t kPlaneLds = 160 * 1024;
+
+// q = t / d for 0 <= t < 2^20 and 0 < d < 2^12, inv = 1 / d in FP32: t + 1/2
+// is at least 1/2 away from any multiple of d, far above the rounding
+__device__ inline int fast_div(int t, float inv) { return int((float(t) + 0.5f) * inv); }
+
+// f(std::integral_constant<int, R>) for a radix 2 <= r <= MAXR (MAXR 12: without
+// 11, whose registers would spill under that kernel's limit of 128)
+template <int MAXR, class F>
+__device__ __forceinline__ void with_radix(int r, F&& f)
+{
+    switch (r) {
+        case 2: f(std::integral_constant<int, 2>{}); break;
+        case 3: f(std::integral_constant<int, 3>{}); break;
+        case 4: f(std::integral_constant<int, 4>{}); break;
+        case 5: f(std::integral_constant<int, 5>{}); break;
+        case 6: f(std::integral_constant<int, 6>{}); break;
+        case 7: f(std::integral_constant<int, 7>{}); break;
+        case 8: f(std::integral_constant<int, 8>{}); break;
+        case 9: f(std::integral_constant<int, 9>{}); break;
+        case 10: f(std::integral_constant<int, 10>{}); break;
+        case 11: if constexpr (MAXR > 12) f(std::integral_constant<int, 11>{}); break;
+        case 12: if constexpr (MAXR >= 12) f(std::integral_constant<int, 12>{}); break;
+        case 13: if constexpr (MAXR >= 13) f(std::integral_constant<int, 13>{}); break;
+        case 14: if constexpr (MAXR >= 14) f(std::integral_constant<int, 14>{}); break;
+        case 15: if constexpr (MAXR >= 15) f(std::integral_constant<int, 15>{}); break;
+        case 16: if constexpr (MAXR >= 16) f(std::integral_constant<int, 16>{}); break;
+        default: break;
+    }
+}
+
+// One axis of the plane in LDS: `lines` lines of n = RA * RB elements,
+// `estr` apart inside a line, consecutive lines `lstr` apart.
+struct PlaneAxis {
+    int n, RA, RB, lines, estr, lstr;
+    float inv_lines, inv_RB;
+    const double2* tw;  // exp(-2 pi i j / n) in LDS
+};
+
+// Forward A step (S = -1: DFT, then the twiddle) or inverse one (S = +1: the
+// conjugate twiddle, then the DFT) from src to dst, each the plane in LDS or
+// in memory with its own element and line strides.  Addresses advance by
+// wave-uniform strides (an index product per element would cost as much as
+// the transform: 32-bit integer multiplies run at a quarter of the FP64 rate).
+template <int NT, int MAXR, int S>
+__device__ __forceinline__ void step_a(const PlaneAxis& ax, int tid, const double2* src, int se, int sl, double2* dst,
+                                       int de, int dl)
+{
+    with_radix<MAXR>(ax.RA, [&](auto r_) {
+        constexpr int R = decltype(r_)::value;
+        const int RB = ax.RB, ntask = ax.lines * RB;
+        for (int t = tid; t < ntask; t += NT) {
+            const int jb = fast_div(t, ax.inv_lines), line = t - jb * ax.lines;
+            const double2* p = src + (line * sl + jb * se);
+            double2* q = dst + (line * dl + jb * de);
+            double2 v[R];
+            sfor<R>([&](auto j_) {
+                constexpr int j = decltype(j_)::value;
+                v[j] = p[j * (RB * se)];
+            });
+            const double2* w = ax.tw;
+            if constexpr (S > 0) {
+                sfor<R - 1>([&](auto j_) {
+                    constexpr int j = decltype(j_)::value + 1;
+                    w += jb;
+                    v[j] = cmul(v[j], cconj(*w));
+                });
+            }
+            reg::rdft<R, S>(v);
+            if constexpr (S < 0) {
+                sfor<R - 1>([&](auto j_) {
+                    constexpr int j = decltype(j_)::value + 1;
+                    w += jb;
+                    v[j] = cmul(v[j], *w);
+                });
+            }
+            sfor<R>([&](auto j_) {
+                constexpr int j = decltype(j_)::value;
+                q[j * (RB * de)] = v[j];
+            });
+        }
+    });
+}
+
+// Forward (S = -1) or inverse (S = +1) B step in place in LDS, or with S = 0
+// both around mul(line, ka, kb, x), the element at frequency ka + RA kb
+template <int NT, int MAXR, int S, class Mul>
+__device__ __forceinline__ void step_b(const PlaneAxis& ax, int tid, double2* pl, Mul mul)
+{
+    with_radix<MAXR>(ax.RB, [&](auto r_) {
+        constexpr int R = decltype(r_)::value;
+        const int ntask = ax.lines * ax.RA;
+        for (int t = tid; t < ntask; t += NT) {
+            const int ka = fast_div(t, ax.inv_lines), line = t - ka * ax.lines;
+            const int es = ax.estr;
+            double2* p = pl + (line * ax.lstr + ka * R * es);
+            double2 u[R];
+            sfor<R>([&](auto j_) {
+                constexpr int j = decltype(j_)::value;
+                u[j] = p[j * es];
+            });
+            reg::rdft<R, S == 0 ? -1 : S>(u);
+            if constexpr (S == 0) {
+                mul(line, ka, u);
+                reg::rdft<R, 1>(u);
+            }
+            sfor<R>([&](auto j_) {
+                constexpr int j = decltype(j_)::value;
+                p[j * es] = u[j];
+            });
+        }
+    });
+}
+
+template <int NT, int MAXR, bool PHASE>
+__global__ void __launch_bounds__(NT, MAXR <= 12 ? 4 : 2) plane_kernel(PlaneArgs a)
+{
+    extern __shared__ double2 lds[];
+    const int N0 = a.N0, N1 = a.N1, N1P = N1 | 1, Nk = N0 * N1;
+    const int tid = threadIdx.x;
+    double2* pl = lds;  // the plane, rows N1P apart
+    double2* tw0 = pl + N0 * N1P;
+    double2* tw1 = tw0 + N0;
+    double2* e0 = tw1 + N1;  // phase: exp(i th R) / n per axis
+    double2* e1 = e0 + N0;
+    for (int i = tid; i < N0; i += NT) tw0[i] = a.tw0[i];
+    for (int i = tid; i < N1; i += NT) tw1[i] = a.tw1[i];
+    // work-groups [0, P) take the first result of their plane, [P, 2P) the
+    // second one (exchange beside the derivative)
+    const int second = blockIdx.x >= unsigned(a.P) ? 1 : 0;
+    const int plane = int(blockIdx.x) - second * a.P;
+    const bool conv = !PHASE && a.conv && (second || !a.out[0]);
+    constexpr bool phase = PHASE;
+    const double2* in = a.in + long(plane) * Nk;
+    double2* out = a.out[conv ? 1 : 0] + long(plane) * Nk;
+    const PlaneAxis x0{N0, a.RA0, a.RB0, N1, N1P, 1, a.inv_N1, a.inv_RB0, tw0};
+    const PlaneAxis x1{N1, a.RA1, a.RB1, N0, 1, N1P, a.inv_N0, 0.f, tw1};
+    // the axis whose B step applies the multiplier, the other one around it.
+    // A derivative along one axis only runs that axis alone: a zero
+    // coefficient adds nothing, wherever it comes from.
+    PlaneAxis in_ax = x1;
+    bool both = true;
+    double dl = 0.0, di = 0.0;  // derivative: coefficients of the outer and the inner axis
+    if (!conv && !phase) {
+        const long inst = a.coef_tab ? plane / a.ppi : 0;
+        const double c0 = a.coef_tab ? a.coef_tab[inst * a.coef_stride] : a.coef[0];
+        const double c1 = a.coef_tab ? a.coef_tab[inst * a.coef_stride + 1] : a.coef[1];
+        // (the same in every lane: kept in scalar registers)
+        const bool use0 = __builtin_amdgcn_readfirstlane(c0 != 0.0), use1 = __builtin_amdgcn_readfirstlane(c1 != 0.0);
+        if (!use0 && !use1) {
+            for (int i = tid; i < Nk; i += NT) out[i] = make_double2(0.0, 0.0);
+            return;
+        }
+        both = use0 && use1;
+        if (both) {
+            dl = c0 / double(N1);
+            di = c1 / double(N0);
+        } else if (use1) {
+            di = c1;
+        } else {
+            di = c0;
+            in_ax = x0;
+            if (in_ax.RB == 1) {  // one step: the one that multiplies
+                in_ax.RB = in_ax.RA;
+                in_ax.RA = 1;
+            }
+        }
+    }
+    if (phase)
+        for (int i = tid; i < N0 + N1; i += NT) {
+            const bool first = i < N0;
+            const int j = first ? i : i - N0, n = first ? N0 : N1;
+            double sn, cs;
+            sincos((first ? a.coef[0] : a.coef[1]) * double(gamma_centred(j, n)), &sn, &cs);
+            const double sc = 1.0 / double(n);
+            (first ? e0 : e1)[j] = make_double2(sc * cs, sc * sn);
+        }
+    const bool copy_in = !both || phase;
+    if (copy_in) {
+        for (int i = tid; i < Nk; i += NT) {
+            double2 v = in[i];
+            if (phase)
+                for (int d = 0; d < 3; ++d) {
+                    if (!a.in_add[d]) continue;
+                    const double2 w = a.in_add[d][long(plane) * Nk + i];
+                    v.x += a.in_add_c[d] * w.x;
+                    v.y += a.in_add_c[d] * w.y;
+                }
+            const int r = fast_div(i, a.inv_N1);
+            pl[r * N1P + (i - r * N1)] = v;
+        }
+    }
+    __syncthreads();  // the twiddles, the phases and a copied plane are in LDS
+    if (both) {
+        if (copy_in)
+            step_a<NT, MAXR, -1>(x0, tid, pl, N1P, 1, pl, N1P, 1);
+        else
+            step_a<NT, MAXR, -1>(x0, tid, in, N1, 1, pl, N1P, 1);
+        __syncthreads();
+        if (x0.RB > 1) {
+            step_b<NT, MAXR, -1>(x0, tid, pl, [](int, int, auto&) {});
+            __syncthreads();
+        }
+    }
+    if (in_ax.RA > 1) {
+        step_a<NT, MAXR, -1>(in_ax, tid, pl, in_ax.estr, in_ax.lstr, pl, in_ax.estr, in_ax.lstr);
+        __syncthreads();
+    }
+    step_b<NT, MAXR, 0>(in_ax, tid, pl, [&](int line, int ka, auto& u) {
+        constexpr int R = sizeof(u) / sizeof(double2);
+        // row position `line` of axis 0 holds frequency f0 after its forward steps
+        const int k0 = fast_div(line, a.inv_RB0), f0 = k0 + a.RA0 * (line - k0 * a.RB0);
+        if (conv) {
+            // zero frequency of both axes: the plane's sum over k
+            if (ka == 0 && line == 0) a.r0[plane] = u[0];
+            const double* W = a.Wp + long(plane) * Nk + (ka * R) * N0 + line;
+            sfor<R>([&](auto k_) {
+                constexpr int k = decltype(k_)::value;
+                u[k] = cscale(u[k], a.conv_scale * W[k * N0]);
+            });
+        } else if (phase) {
+            const double2 p0 = e0[f0];
+            sfor<R>([&](auto k_) {
+                constexpr int k = decltype(k_)::value;
+                u[k] = cmul(u[k], cmul(p0, e1[ka + x1.RA * k]));
+            });
+        } else {
+            const double r0 = dl * double(gamma_centred(f0, N0));
+            sfor<R>([&](auto k_) {
+                constexpr int k = decltype(k_)::value;
+                u[k] = cmul_i(u[k], r0 + di * double(gamma_centred(ka + in_ax.RA * k, in_ax.n)));
+            });
+        }
+    });
+    __syncthreads();
+    if (in_ax.RA > 1) {
+        step_a<NT, MAXR, 1>(in_ax, tid, pl, in_ax.estr, in_ax.lstr, pl, in_ax.estr, in_ax.lstr);
+        __syncthreads();
+    }
+    if (both) {
+        if (x0.RB > 1) {
+            step_b<NT, MAXR, 1>(x0, tid, pl, [](int, int, auto&) {});
+            __syncthreads();
+        }
+        step_a<NT, MAXR, 1>(x0, tid, pl, N1P, 1, out, N1, 1);
+    } else {
+        for (int i = tid; i < Nk; i += NT) {
+            const int r = fast_div(i, a.inv_N1);
+            out[i] = pl[r * N1P + (i - r * N1)];
+        }
+    }
+}
+
+// W[f0 * N1 + f1] of every plane into the order the convolution reads it:
+// Wp[p1 * N0 + p0], the frequencies at positions p0, p1 of the two axes
+__global__ void plane_permute_kernel(const double* __restrict__ W, double* __restrict__ Wp, long total, int N0, int N1,
+                                     int RA0, int RB0, int RA1, int RB1)
+{
+    const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= total) return;
+    const int Nk = N0 * N1;
+    const long p = i / Nk;
+    const int e = int(i - p * Nk), p1 = e / N0, p0 = e - p1 * N0;
+    const int f0 = p0 / RB0 + RA0 * (p0 % RB0), f1 = p1 / RB1 + RA1 * (p1 % RB1);
+    Wp[i] = W[p * Nk + long(f0) * N1 + f1];
+}
+
+// n = RA * RB with both at most 16, the larger factor as small as possible;
+// lines of at most 16 are one step
+bool split_line(int n, int& big, int& small)
+{
+    if (n < 2) return false;
+    if (n <= 16) {
+        big = n;
+        small = 1;
+        return true;
+    }
+    for (big = 2; big <= 16; ++big)
+        if (n % big == 0 && n / big <= big) {
+            small = n / big;
+            return true;
+        }
+    return false;
+}
+
+template <int NT, int MAXR, bool PHASE>
+void launch_plane_nt(const PlaneArgs& a, int blocks, size_t lds, hipStream_t s)
+{
+    auto kern = &plane_kernel<NT, MAXR, PHASE>;
+    static std::once_flag raised;  // contexts may be created from several host threads
+    std::call_once(raised, [&] {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  int(kPlaneLds));
+    });
+    if (g_attributes_only) return;
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), lds, s, a);
+}
+
+size_t plane_lds(int N0, int N1, bool phase)
+{
+    return size_t(N0 * (N1 | 1) + (phase ? 2 : 1) * (N0 + N1)) * sizeof(double2);
+}
+
+}  // namespace
+
+bool plane_available(int N0, int N1)
+{
+    int b, c;
+    return split_line(N0, b, c) && split_line(N1, b, c) && plane_lds(N0, N1, true) <= kPlaneLds;
+}
+
+PlaneArgs plane_args(int N0, int N1)
+{
+    PlaneArgs a{};
+    a.N0 = N0;
+    a.N1 = N1;
+    split_line(N0, a.RA0, a.RB0);
+    // the inner axis keeps the multiplier in its B step
+    if (N1 <= 16) {
+        a.RA1 = 1;
+        a.RB1 = N1;
+    } else {
+        split_line(N1, a.RA1, a.RB1);
+    }
+    a.inv_N0 = 1.0f / float(N0);
+    a.inv_N1 = 1.0f / float(N1);
+    a.inv_RB0 = 1.0f / float(a.RB0);
+    return a;
+}
+
+template <bool PHASE>
+void launch_plane_shape(const PlaneArgs& a, hipStream_t s)
+{
+    const int blocks = a.P * (PHASE ? 1 : (a.out[0] ? 1 : 0) + (a.conv ? 1 : 0));
+    const size_t lds = plane_lds(a.N0, a.N1, PHASE);
+    // 11 and radices above 12 need more than 128 registers.  The others run with
+    // as many threads as give a step about one round of tasks (us for 256, 512,
+    // 1024 threads: 30 x 30, 4 planes 6.2, 6.2, 6.5; 60 x 66, 25 planes 13.7,
+    // 11.9, 12.2; 90 x 90 with exchange, 64 planes 25.0, 22.1, 18.9)
+    bool wide = false;
+    for (int r : {a.RA0, a.RB0, a.RA1, a.RB1}) wide = wide || r > 12 || r == 11;
+    const int Nk = a.N0 * a.N1;
+    if (wide)
+        launch_plane_nt<512, 16, PHASE>(a, blocks, lds, s);
+    else if (Nk <= 1024)
+        launch_plane_nt<256, 12, PHASE>(a, blocks, lds, s);
+    else if (Nk <= 6000)
+        launch_plane_nt<512, 12, PHASE>(a, blocks, lds, s);
+    else
+        launch_plane_nt<1024, 12, PHASE>(a, blocks, lds, s);
+}
+
+void launch_plane(const PlaneArgs& a, hipStream_t s)
+{
+    if (a.phase)
+        launch_plane_shape<true>(a, s);
+    else
+        launch_plane_shape<false>(a, s);
+}
+
+void launch_plane_permute(const double* W, double* Wp, int P, int N0, int N1, hipStream_t s)
+{
+    const PlaneArgs a = plane_args(N0, N1);
+    const long n = long(P) * N0 * N1;
+    hipLaunchKernelGGL(plane_permute_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, W, Wp, n, N0, N1, a.RA0,
+                       a.RB0, a.RA1, a.RB1);
+}
+
+}  // namespace edus

@@ -198,7 +198,9 @@ int edus_graph(edus_ctx* ctx, int steps_per_graph);
  * launch of the named kernel class is bracketed by events; edus_timing_get
  * returns the summed milliseconds and launch count since the last reset.
  * Classes: "grad_col", "grad_row", "grad_fused", "kgrad", "comm", "hf_row",
- * "hf_col", "peierls_col", "peierls_row", "rotate". */
+ * "hf_col", "hf_plane" (the exchange term, with the derivative where the field
+ * has one, one work-group per plane), "peierls_col", "peierls_row",
+ * "peierls_plane", "rotate". */
 int edus_timing_enable(edus_ctx* ctx, int on);
 int edus_timing_get(edus_ctx* ctx, const char* kernel_class, double* total_ms, long* count);
 
@@ -219,8 +221,11 @@ int edus_timing_get(edus_ctx* ctx, const char* kernel_class, double* total_ms, l
  *   comm_tile_ab   the same for the Adams-Bashforth steps
  *   grad_fused     1: the spectral derivative in one pass per plane (one
  *                  work-group holds a plane: grids 120 x 120, 96 x 96,
- *                  90 x 90, 48 x 48); 0: two axis passes through a work plane
- *                  set.  Used when the field has components along both axes.
+ *                  90 x 90, 48 x 48; on the last three the exchange term too);
+ *                  0: axis passes through work plane sets.  Other grids have
+ *                  no choice (0): with exchange, or where an axis has no
+ *                  two-step kernel, planes that fit in LDS go one work-group
+ *                  per plane, the rest take axis passes.
  *   tri_fields     1: the MFMA commutator engines read H0(k) and r_d(k) from
  *                  copies of their upper triangles, the lower elements as
  *                  conjugates (0.54 of the bytes at nb = 14); 0: from every
