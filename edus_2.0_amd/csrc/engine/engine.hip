@@ -202,7 +202,6 @@ Engine::Engine(const edus_desc& d, const EngineOptions& opt)
     alloc(reinterpret_cast<void**>(&mon), kMonWords * sizeof(unsigned long long));
     const int nv = 2 * nb + 6;
     alloc(reinterpret_cast<void**>(&obs_partial), size_t(observables_blocks(Nk)) * nv * sizeof(double));
-    alloc(reinterpret_cast<void**>(&obs_out), size_t(nv) * sizeof(double));
 
     upload(d.H0k, H0);
     for (int k = 0; k < 3; ++k) {
@@ -411,18 +410,14 @@ void Engine::observables(double* pop_bloch, double* pop_wannier, double* vel_out
     a.Nk = Nk;
     a.layout = layout;
     a.rho = rho_override ? rho_override : y + io;
-    a.rho_bloch = nullptr;
-    if (U) {  // Bloch populations from U^dagger rho U (Simulation.cpp:439-470), staged in full planes
-        rotate(a.rho, stage, kFull, true, inst);
-        a.rho_bloch = stage;
-    }
+    a.U = U ? U + size_t(inst) * nb * nb * Nk : nullptr;  // Bloch populations from U^dagger rho U (Simulation.cpp:439-470)
     for (int d = 0; d < 3; ++d) a.vel[d] = vel[d] ? vel[d] + io : nullptr;
     a.partial = obs_partial;
-    launch_observables(a, obs_out, s);
     const int nv = 2 * nb + 6;
-    std::vector<double> h(nv);
-    HIP_CHECK(hipMemcpyAsync(h.data(), obs_out, nv * sizeof(double), hipMemcpyDeviceToHost, s));
+    if (!obs_out) HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&obs_out), nv * sizeof(double)));
+    launch_observables(a, prec == EDUS_PREC_MIXED ? kCommMfma32 : kCommMfma64, obs_out, s);
     HIP_CHECK(hipStreamSynchronize(s));
+    const double* h = obs_out;
     for (int n = 0; n < nb; ++n) {
         if (pop_bloch) pop_bloch[n] = U ? ((n < nf) ? 1. - h[n] : h[n]) : 0.0;  // Simulation.cpp:459-465
         if (pop_wannier) pop_wannier[n] = h[nb + n];
@@ -477,6 +472,7 @@ Engine::~Engine()
         (void)hipEventDestroy(e.b);
     }
     for (void* p : owned) (void)hipFree(p);
+    if (obs_out) (void)hipHostFree(obs_out);
     if (s) (void)hipStreamDestroy(s);
 }
 
@@ -1150,7 +1146,6 @@ Engine::Engine(const std::vector<const Engine*>& members)
     alloc(reinterpret_cast<void**>(&mon), kMonWords * sizeof(unsigned long long));
     const int nv = 2 * nb + 6;
     alloc(reinterpret_cast<void**>(&obs_partial), size_t(observables_blocks(Nk)) * nv * sizeof(double));
-    alloc(reinterpret_cast<void**>(&obs_out), size_t(nv) * sizeof(double));
 
     // stacked copies of every member's arrays (zero where a member has none)
     auto stack = [&](double2* dst, auto get, size_t bytes) {

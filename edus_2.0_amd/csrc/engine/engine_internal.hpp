@@ -131,7 +131,7 @@ class Engine {
     bool plane_exchange() const { return plane_ok && (kgrad || !grad_form_choice(N0, N1) || grad_fused); }
     double2 *hdiag = nullptr, *hsum = nullptr;  // hdiag: set-up only
     int force_kind = -1;  // >= 0: the autotuner keeps this commutator engine (batch groups)
-    double *obs_partial = nullptr, *obs_out = nullptr;
+    double *obs_partial = nullptr, *obs_out = nullptr;  // obs_out: pinned host memory
     unsigned long long* mon = nullptr;
     double2* hist[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
     int abidx[5] = {0, 1, 2, 3, 4};

@@ -82,52 +82,21 @@ __global__ void full_to_planes_kernel(const double2* __restrict__ full, double2*
     planes[idx] = full[long(k) * nb2 + q];
 }
 
-constexpr int kObsBlock = 128;  // keeps the (2nb+6) x block LDS tile of the observables kernel <= 38 KB
+constexpr int kObsBlock = 128;
 
-// Per-block partial sums of the observables over k:
-//   vals[0..nb)       sum_k Re (U^dagger rho U)_nn      (Bloch population, from the rotated field)
-//   vals[nb..2nb)     sum_k Re rho_nn                    (Wannier population)
-//   vals[2nb..2nb+6)  sum_k Tr(V_d rho)  (re, im per d)
-__global__ void __launch_bounds__(kObsBlock) observables_kernel(ObsArgs a)
+// out[v] = scale * the sum of partial[v][0..nblocks), in a fixed order: one wave
+// per value, its lanes over the partial sums
+__global__ void __launch_bounds__(1024) reduce_partials_kernel(const double* __restrict__ partial, int nblocks, int nv,
+                                                               double scale, double* __restrict__ out)
 {
-    const int nb = a.nb, Nk = a.Nk, L = a.layout;
-    const int nv = 2 * nb + 6;
-    extern __shared__ double sh[];  // [nv][kObsBlock]
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    for (int v = 0; v < nv; ++v) sh[v * kObsBlock + threadIdx.x] = 0.;
-    if (k < Nk) {
-        for (int n = 0; n < nb; ++n) sh[(nb + n) * kObsBlock + threadIdx.x] = element(a.rho, n, n, nb, L, Nk, k).x;
-        if (a.rho_bloch)
-            for (int n = 0; n < nb; ++n) sh[n * kObsBlock + threadIdx.x] = a.rho_bloch[long(n * nb + n) * Nk + k].x;
-        for (int d = 0; d < 3; ++d) {
-            if (!a.vel[d]) continue;
-            double2 tr = make_double2(0., 0.);
-            for (int i = 0; i < nb; ++i)
-                for (int j = 0; j < nb; ++j)
-                    tr = cadd(tr, cmul(element(a.vel[d], i, j, nb, L, Nk, k), element(a.rho, j, i, nb, L, Nk, k)));
-            sh[(2 * nb + 2 * d) * kObsBlock + threadIdx.x] = tr.x;
-            sh[(2 * nb + 2 * d + 1) * kObsBlock + threadIdx.x] = tr.y;
-        }
+    const int lane = threadIdx.x & 63;
+    for (int v = threadIdx.x >> 6; v < nv; v += blockDim.x >> 6) {
+        double s = 0.;
+        for (int b = lane; b < nblocks; b += 64) s += partial[long(v) * nblocks + b];
+#pragma unroll
+        for (int w = 32; w > 0; w >>= 1) s += __shfl_xor(s, w);
+        if (lane == 0) out[v] = s * scale;
     }
-    __syncthreads();
-    for (int s = kObsBlock / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s)
-            for (int v = 0; v < nv; ++v) sh[v * kObsBlock + threadIdx.x] += sh[v * kObsBlock + threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        for (int v = 0; v < nv; ++v) a.partial[long(blockIdx.x) * nv + v] = sh[v * kObsBlock];
-}
-
-// Deterministic final reduction of per-block partials (fixed order).
-__global__ void reduce_partials_kernel(const double* __restrict__ partial, int nblocks, int nv, double scale,
-                                       double* __restrict__ out)
-{
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nv) return;
-    double s = 0.;
-    for (int b = 0; b < nblocks; ++b) s += partial[long(b) * nv + v];
-    out[v] = s * scale;
 }
 
 // hdiag = Hartree shift of B stacked instances from their plane sums over k
@@ -246,15 +215,12 @@ void launch_full_to_planes(const double2* full, double2* planes, int nb, int Nk,
     hipLaunchKernelGGL(full_to_planes_kernel, dim3(grid1d(long(nb) * nb * Nk, 256)), dim3(256), 0, s, full, planes,
                        nb * nb, Nk);
 }
-int observables_blocks(int Nk) { return int(grid1d(Nk, kObsBlock)); }
-void launch_observables(const ObsArgs& a, double* out, hipStream_t s)
+void launch_observables(const ObsArgs& a, int kind, double* out, hipStream_t s)
 {
     const int nv = 2 * a.nb + 6;
-    const int blocks = observables_blocks(a.Nk);
-    hipLaunchKernelGGL(observables_kernel, dim3(blocks), dim3(kObsBlock), size_t(nv) * kObsBlock * sizeof(double), s,
-                       a);
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(64), 0, s, a.partial, blocks, nv, 1.0 / double(a.Nk),
-                       out);
+    launch_observe_partials(a, kind, s);
+    hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(1024), 0, s, a.partial, observables_blocks(a.Nk), nv,
+                       1.0 / double(a.Nk), out);
 }
 void launch_hartree_sums(const double2* hsum, const double* hart, int nb, int layout, int P, int B, double inv_nk,
                          double2* hdiag, hipStream_t s)

@@ -26,6 +26,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "obs.hpp"
 
 namespace edus {
 
@@ -241,7 +242,211 @@ void launch_rot_nb(const RotateArgs& a, int in_layout, int kind, hipStream_t s)
     }
 }
 
+// The observables of the state, sums over k of
+//   vals[0..nb)       Re (U^dagger rho U)_nn      (Bloch populations; U may be null)
+//   vals[nb..2nb)     Re rho_nn                   (Wannier populations)
+//   vals[2nb..2nb+6)  Tr(V_d rho)                 (re, im per d)
+// (Simulation.cpp:439-470,583-622), one partial sum per work-group.  A tile of
+// 8 k-points is loaded and rotated as in rotate_kernel (the same products, so
+// the populations of a k-point are the rotated field's diagonal bit for bit),
+// but nothing is written back: the diagonal is summed from the matrix cores'
+// result registers, and the velocity operators meet the tile of rho in LDS.
+// A work-group takes every gridDim.x-th tile.  Bound by the read of rho, U and
+// the V_d: nb = 14, 120 x 120, two V_d: 181 MB.  The rotated field stored and
+// read back with one thread per k-point summing nb^2 terms took 275 us.
+template <int NB, int LAYOUT, int KIND>
+__global__ void __launch_bounds__(kRotThreads) observe_kernel(ObsArgs a)
+{
+    constexpr int NPL = rot_npl<NB, LAYOUT>();
+    constexpr int M = NB * NB;
+    constexpr int SA = rot_slots(NPL) > rot_slots(M) ? rot_slots(NPL) : rot_slots(M);
+    constexpr int PER = (NPL * kRotTK + kRotThreads - 1) / kRotThreads;
+    constexpr int NV = 2 * NB + 6, NW = kRotThreads / 64;
+    using acc_t = typename std::conditional<KIND == kCommMfma64, dbl4, flt4>::type;
+    extern __shared__ double2 lds[];
+    double2* sO = lds;
+    double2* sU = lds + SA;
+    const int Nk = a.Nk;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int kk = wave, i = lane & 15, q = lane >> 4;
+    const int ntile = (Nk + kRotTK - 1) / kRotTK;
+    double pb = 0.0, pw = 0.0;  // this lane's share of band i
+    double2 tr[3] = {make_double2(0., 0.), make_double2(0., 0.), make_double2(0., 0.)};
+    for (int t = blockIdx.x; t < ntile; t += gridDim.x) {
+        const int k0 = t * kRotTK;
+        for (int c = wave; c < rot_slots(NPL) / 64; c += NW) {
+            const int s = c * 64 + lane, p = s / kRotPS, kt = s - p * kRotPS;
+            if (kt < kRotTK && p < NPL && k0 + kt < Nk)
+                __builtin_amdgcn_global_load_lds(a.rho + long(p) * Nk + k0 + kt, sO + c * 64, 16, 0, 0);
+        }
+        if (a.U)
+            for (int c = wave; c < rot_slots(M) / 64; c += NW) {
+                const int s = c * 64 + lane, p = s / kRotPS, kt = s - p * kRotPS;
+                if (kt < kRotTK && p < M && k0 + kt < Nk)
+                    __builtin_amdgcn_global_load_lds(a.U + long(p) * Nk + k0 + kt, sU + c * 64, 16, 0, 0);
+            }
+        double2 v[3][PER];
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                const int e = threadIdx.x + j * kRotThreads, p = e / kRotTK, kt = e - p * kRotTK;
+                v[d][j] = make_double2(0., 0.);
+                if (a.vel[d] && e < NPL * kRotTK && k0 + kt < Nk) v[d][j] = a.vel[d][long(p) * Nk + k0 + kt];
+            }
+        __builtin_amdgcn_s_waitcnt(0);  // this wave's direct loads are in LDS
+        __syncthreads();                // and every other wave's
+        // Tr(V rho) = sum_nm V_nm rho_mn over this thread's elements; HERMITIAN:
+        // the pair n < m adds V_nm conj(rho_nm) and its conjugate
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int e = threadIdx.x + j * kRotThreads, p = e / kRotTK, kt = e - p * kRotTK;
+            if (e >= NPL * kRotTK || k0 + kt >= Nk) continue;
+            int n, m;
+            if (LAYOUT == kFull) {
+                n = p / NB;
+                m = p - n * NB;
+            } else {
+                n = 0;
+                int r = p;
+                while (r >= NB - n) {
+                    r -= NB - n;
+                    ++n;
+                }
+                m = n + r;
+            }
+            const double2 x = in_elem<NB, LAYOUT>(sO, m, n, kt);
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const double2 w = cmul(v[d][j], x);
+                if (LAYOUT == kFull || n == m)
+                    tr[d] = cadd(tr[d], w);
+                else
+                    tr[d].x += 2.0 * w.x;
+            }
+        }
+        const bool valid = k0 + kk < Nk;
+        if (valid && q == 0 && i < NB) pw += in_elem<NB, LAYOUT>(sO, i, i, kk).x;
+        if (a.U) {
+            acc_t cr{}, ci{};
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {  // T = U^dagger rho
+                if (4 * s >= NB) break;
+                const int c = 4 * s + q;
+                double2 A = full_elem<NB>(sU, c, i, kk);
+                A.y = -A.y;
+                cgemm_step<KIND>(A, in_elem<NB, LAYOUT>(sO, c, i, kk), cr, ci);
+            }
+            __syncthreads();  // every wave has read rho before T replaces it
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+                const int r = result_row<KIND>(q, r4);
+                if (r < NB && i < NB)
+                    sO[(r * NB + i) * kRotPS + kk] = make_double2(double(cr[r4]), double(ci[r4]));
+            }
+            __syncthreads();
+            cr = acc_t{};
+            ci = acc_t{};
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {  // T U
+                if (4 * s >= NB) break;
+                const int c = 4 * s + q;
+                cgemm_step<KIND>(full_elem<NB>(sO, i, c, kk), full_elem<NB>(sU, c, i, kk), cr, ci);
+            }
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4)
+                if (valid && result_row<KIND>(q, r4) == i && i < NB) pb += double(cr[r4]);
+        }
+        __syncthreads();  // every wave is done with the tile
+    }
+    // across the lane groups of a band, then the waves, in a fixed order
+    double* red = reinterpret_cast<double*>(lds);  // [NW][NV]
+#pragma unroll
+    for (int w = 32; w >= 16; w >>= 1) {
+        pb += __shfl_xor(pb, w);
+        pw += __shfl_xor(pw, w);
+    }
+    if (q == 0 && i < NB) {
+        red[wave * NV + i] = pb;
+        red[wave * NV + NB + i] = pw;
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+#pragma unroll
+        for (int w = 32; w > 0; w >>= 1) {
+            tr[d].x += __shfl_xor(tr[d].x, w);
+            tr[d].y += __shfl_xor(tr[d].y, w);
+        }
+        if (lane == 0) {
+            red[wave * NV + 2 * NB + 2 * d] = tr[d].x;
+            red[wave * NV + 2 * NB + 2 * d + 1] = tr[d].y;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < NV) {
+        double s = 0.0;
+        for (int w = 0; w < NW; ++w) s += red[w * NV + threadIdx.x];
+        a.partial[long(threadIdx.x) * gridDim.x + blockIdx.x] = s;
+    }
+}
+
+template <int NB, int LAYOUT, int KIND>
+void launch_observe(const ObsArgs& a, hipStream_t s)
+{
+    constexpr size_t lds = rot_lds_bytes<NB, LAYOUT>() > 8 * (2 * NB + 6) * sizeof(double)
+                               ? rot_lds_bytes<NB, LAYOUT>()
+                               : 8 * (2 * NB + 6) * sizeof(double);
+    auto kern = &observe_kernel<NB, LAYOUT, KIND>;
+    static std::once_flag raised;  // contexts may be created from several host threads
+    std::call_once(raised, [&] {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  int(lds));
+    });
+    hipLaunchKernelGGL(kern, dim3(observables_blocks(a.Nk)), dim3(kRotThreads), lds, s, a);
+}
+
+template <int NB>
+void launch_observe_nb(const ObsArgs& a, int kind, hipStream_t s)
+{
+    if (a.layout == kFull) {
+        if (kind == kCommMfma32)
+            launch_observe<NB, kFull, kCommMfma32>(a, s);
+        else
+            launch_observe<NB, kFull, kCommMfma64>(a, s);
+    } else {
+        if (kind == kCommMfma32)
+            launch_observe<NB, kHermitian, kCommMfma32>(a, s);
+        else
+            launch_observe<NB, kHermitian, kCommMfma64>(a, s);
+    }
+}
+
 }  // namespace
+
+int observables_blocks(int Nk) { return std::min((Nk + kRotTK - 1) / kRotTK, 512); }
+
+void launch_observe_partials(const ObsArgs& a, int kind, hipStream_t s)
+{
+    switch (a.nb) {
+        case 1: launch_observe_nb<1>(a, kind, s); break;
+        case 2: launch_observe_nb<2>(a, kind, s); break;
+        case 3: launch_observe_nb<3>(a, kind, s); break;
+        case 4: launch_observe_nb<4>(a, kind, s); break;
+        case 5: launch_observe_nb<5>(a, kind, s); break;
+        case 6: launch_observe_nb<6>(a, kind, s); break;
+        case 7: launch_observe_nb<7>(a, kind, s); break;
+        case 8: launch_observe_nb<8>(a, kind, s); break;
+        case 9: launch_observe_nb<9>(a, kind, s); break;
+        case 10: launch_observe_nb<10>(a, kind, s); break;
+        case 11: launch_observe_nb<11>(a, kind, s); break;
+        case 12: launch_observe_nb<12>(a, kind, s); break;
+        case 13: launch_observe_nb<13>(a, kind, s); break;
+        case 14: launch_observe_nb<14>(a, kind, s); break;
+        case 15: launch_observe_nb<15>(a, kind, s); break;
+        case 16: launch_observe_nb<16>(a, kind, s); break;
+        default: break;  // rejected at context creation
+    }
+}
 
 void launch_rotate(int nb, int in_layout, int kind, const RotateArgs& a, hipStream_t s)
 {
