@@ -11,9 +11,11 @@
 //   X_ab(q) = 1/Nk sum_k sum_c B_c(k+q)_ab sum_v r_vc(k, k+q) A_v(k)_ab,
 //   r_vc(k, k') = 1 / (e_v(k) - e_c(k')).
 //
-// The sum is elementwise in (a, b): no contraction that matrix cores could
-// take, and O(Nk^2) pairs (q, k) with O(nb^2 nv nc) FP64 work each, so the
-// kernel is bound by the FP64 vector pipes, not by HBM.  Mapping:
+// O(Nk^2) pairs (q, k) with O(nb^2 nv nc) FP64 work each: the kernels are bound
+// by the FP64 pipes and what feeds them, not by HBM.  Two forms follow: this
+// one on the vector pipes, elementwise in (a, b), and one that takes the sum
+// over v on the matrix cores (below); lindhard_mfma_shape chooses.  Mapping of
+// the vector form:
 //   * a split pass stores the valence columns of every U_k as Uv[k][v][a]
 //     and the conduction columns as planes Uc[c nb + a][k], so that a step's
 //     valence block is one contiguous run and the conduction elements of the
@@ -44,6 +46,7 @@
 // of bands, r multiplied instead of divided), so results agree to rounding,
 // not bit for bit.
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -61,6 +64,7 @@ namespace {
 
 constexpr int kLindStageR = 4;  // reciprocals formed per thread per k
 constexpr int kLindGatherU = 8;  // conduction-column elements gathered per thread per k
+typedef double dbl4 __attribute__((ext_vector_type(4)));
 
 struct LindhardArgs {
     const double2* Uv;  // [Nk][nv][nb]: U_k(a, v) at (k nv + v) nb + a
@@ -357,7 +361,10 @@ void launch_nv(const LindhardArgs& a0, int blocks, size_t lds, hipStream_t s)
     const long cap = long(std::max(per_cu, 1)) * std::max(ncu, 1);
     auto fill = [&](long n) { return double(n) / double(((n + cap - 1) / cap) * cap); };
     a.KS = (a.Nk >= 64 && fill(2L * blocks) > fill(blocks) + 0.05) ? 2 : 1;
-    if (a.KS > 1) EDUS_HIP_CHECK(hipMemsetAsync(a.X, 0, size_t(a.nb) * a.nb * a.Nk * sizeof(double2), s));
+    if (a.KS > 1) {  // a kernel: callers may capture this
+        const long n = long(a.nb) * a.nb * a.Nk;
+        hipLaunchKernelGGL(lindhard_zero_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, a.X, n);
+    }
     hipLaunchKernelGGL(kern, dim3(blocks * a.KS), dim3(64 * a.W), lds, s, a);
 }
 
@@ -372,6 +379,434 @@ void launch_tq(const LindhardArgs& a, int blocks, size_t lds, hipStream_t s)
 #undef EDUS_NV
         default: throw EngineError(EDUS_ERR_ARG, "lindhard: filled bands out of range");
     }
+}
+
+// ---- the matrix-core form
+//
+// For one k and the (q, c) rows of 4 consecutive q and 4 conduction bands, the
+// inner sum S_c(q)_ab = sum_v r_vc(k, k+q) A_v(k)_ab is a 16 x nv by nv x 16
+// real product (real and imaginary part of A) for every 16 element pairs:
+// v_mfma_f64_16x16x4.  The FP64 matrix cores and the vector pipes share their
+// rate on this chip, so the products cost what they cost in vector FMAs (less
+// the padding of nv and nc to multiples of 4); what the matrix form saves is
+// LDS bandwidth, which bounds the vector form: there every lane reads every
+// r_vc from LDS, here a lane reads one per 16 x 16 products.  Result slot v of
+// lane group g is row g + 4 v = (q g, c v), so each lane accumulates X(q)_ab
+// over c and k in its own registers.
+//   * a work-group takes GT consecutive q of one grid row (and a range of k
+//     rows) and walks k along each row: k + q then slides by one point per
+//     step, and B_c(k')_ab = conj U_k'(a,c) U_k'(b,c) is formed once per
+//     point, into a ring of GT + 1 slots, instead of once per (k, q);
+//   * A_v(k) and the reciprocals of step k + 1 are formed from registers loaded
+//     one step ahead while step k multiplies; one barrier per step;
+//   * units of (4 q, 16 pairs) are dealt to the waves, at most UPW each;
+//   * parts of the k range are summed by a second kernel, in a fixed order.
+struct LindhardMfmaArgs {
+    const double2* U;    // [Nk][nb][nb], bands in columns
+    const double* eps;   // [Nk][nb]
+    double2* X;          // planes [nb * nb][Nk]
+    double2* work;       // another nb * nb planes, for partial sums
+    int nb, nv, nc, N0, N1, Nk;
+    int P, T;            // element pairs a <= b, tiles of 16
+    int GT, KS, nqb_row;
+    double inv_nk;
+};
+
+// where part ks of the sum for pair p, point q is kept (parts 0 and 1 in the
+// first P planes of X and work, part 2 in the planes these leave, P <= 2 (nb^2 - P))
+__device__ inline double2* lindhard_part(const LindhardMfmaArgs& a, int ks, int p, int q)
+{
+    const int left = a.nb * a.nb - a.P;
+    if (ks == 0) return a.X + long(p) * a.Nk + q;
+    if (ks == 1) return a.work + long(p) * a.Nk + q;
+    return (p < left ? a.X + long(a.P + p) * a.Nk : a.work + long(a.P + p - left) * a.Nk) + q;
+}
+
+// LDS of the matrix-core kernel: the ring of B, two of A and two tables of r
+struct LindhardMfmaLds {
+    int ring, A, r;  // entries of one ring slot, one A buffer (double2), one r table (double)
+    __host__ __device__ LindhardMfmaLds(int nv, int nc, int T, int GT)
+    {
+        const int cv = (nv + 3) / 4 * 4, cc = (nc + 3) / 4 * 4;
+        ring = nc * 16 * T;
+        A = cv * 16 * T;
+        r = GT * cc * cv;
+    }
+    __host__ __device__ int elems(int GT) const { return (GT + 1) * ring + 2 * A + (2 * r + 1) / 2; }
+};
+
+// Threads, and products A_v (n = CV) or B_c (n = CC) per thread and step, by the
+// numbers of valence and conduction quadruples, nb <= 4 (CV + CC) and nb <= 16
+constexpr int lind_threads(int CV, int CC) { return CV + CC <= 3 ? 256 : 512; }
+// (at most 16 * 17 / 2 pairs times 4 n bands, n quadruples)
+constexpr int lind_items(int n, int CV, int CC)
+{
+    const int nb = 4 * (CV + CC) < 16 ? 4 * (CV + CC) : 16, bands = 4 * n < nb ? 4 * n : nb - 1;
+    return (nb * (nb + 1) / 2 * bands + lind_threads(CV, CC) - 1) / lind_threads(CV, CC);
+}
+
+template <int CV, int CC, int UPW>
+__global__ void __launch_bounds__(lind_threads(CV, CC)) lindhard_mfma_kernel(LindhardMfmaArgs a)
+{
+    constexpr int NT = lind_threads(CV, CC), NA = lind_items(CV, CV, CC), NB = lind_items(CC, CV, CC);
+    extern __shared__ double2 lds[];
+    const int nb = a.nb, nv = a.nv, nc = a.nc, N0 = a.N0, N1 = a.N1, P = a.P, T = a.T, GT = a.GT;
+    const int Pp = 16 * T;
+    const LindhardMfmaLds sz(nv, nc, T, GT);
+    double2* ring = lds;
+    double2* bufA = ring + (GT + 1) * sz.ring;
+    double* bufR = reinterpret_cast<double*>(bufA + 2 * sz.A);
+    const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int L = xcd_contiguous_block();
+    const int qb = L / a.KS, ks = L - qb * a.KS;
+    const int q0 = qb / a.nqb_row, q1f = (qb - q0 * a.nqb_row) * GT;
+    const int row_b = N0 * ks / a.KS, row_e = N0 * (ks + 1) / a.KS;
+    // padded bands and pairs are zero in every buffer and never written again
+    for (int e = tid; e < sz.elems(GT); e += NT) lds[e] = make_double2(0.0, 0.0);
+
+    // products of this thread, A_v(k)_ab = U(a,v) conj U(b,v) and, at the point
+    // that enters the window, B_c_ab = conj U(a,c) U(b,c): offsets of the two
+    // factors in a point's matrix and of the result in its buffer
+    int a1[NA], a2[NA], ad[NA], b1[NB], b2[NB], bd[NB];
+    auto items = [&](int bands, int first, auto& o1, auto& o2, auto& od) {
+        constexpr int N = sizeof(od) / sizeof(int);
+#pragma unroll
+        for (int t = 0; t < N; ++t) {
+            const int e = tid + t * NT;
+            const bool use = e < P * bands;
+            const int n = use ? e / P : 0, p = use ? e - n * P : 0;
+            int al, be;
+            pair_of(p, nb, 1, al, be);
+            o1[t] = al * nb + first + n;
+            o2[t] = be * nb + first + n;
+            od[t] = use ? n * Pp + p : -1;
+        }
+    };
+    items(nv, 0, a1, a2, ad);
+    items(nc, nv, b1, b2, bd);
+    // reciprocals of this thread: (slot, c, v) of the GT x nc x nv
+    constexpr int NR = 2;
+    int rv[NR], rc[NR], rs[NR], rd[NR];
+#pragma unroll
+    for (int t = 0; t < NR; ++t) {
+        const int e = tid + t * NT;
+        rd[t] = -1;
+        rv[t] = rc[t] = rs[t] = 0;
+        if (e < GT * nc * nv) {
+            rs[t] = e / (nc * nv);
+            const int m = e - rs[t] * nc * nv;
+            rc[t] = m / nv;
+            rv[t] = m - rc[t] * nv;
+            rd[t] = (rs[t] * 4 * CC + rc[t]) * 4 * CV + rv[t];
+        }
+    }
+    // the wave's units: q group and tile (a wave with fewer repeats unit 0 and
+    // drops the result: no branch between units, whose loads then overlap)
+    int uq[UPW], ut[UPW];
+    bool uok[UPW];
+#pragma unroll
+    for (int u = 0; u < UPW; ++u) {
+        const int n = wave + u * (NT / 64);
+        uok[u] = n < (GT / 4) * T;
+        uq[u] = uok[u] ? n / T : 0;
+        ut[u] = uok[u] ? n - uq[u] * T : 0;
+    }
+    double2 acc[UPW];
+    int oA[UPW], oR[UPW];  // this lane's operands of the first quadruple in a buffer of A and a table of r
+#pragma unroll
+    for (int u = 0; u < UPW; ++u) {
+        acc[u] = make_double2(0.0, 0.0);
+        oA[u] = g * Pp + 16 * ut[u] + i;
+        oR[u] = ((4 * uq[u] + (i & 3)) * 4 * CC + (i >> 2)) * 4 * CV + g;
+    }
+    // offsets of the conduction bands in a ring slot; the bands that pad the
+    // last quadruple repeat the last one (their rows of r are zero)
+    int oc[4 * CC];
+#pragma unroll
+    for (int c = 0; c < 4 * CC; ++c) oc[c] = min(c, nc - 1) * Pp;
+    const int ring_end = (GT + 1) * sz.ring;
+
+    for (int k0 = row_b; k0 < row_e; ++k0) {
+        int r0 = k0 + q0;
+        if (r0 >= N0) r0 -= N0;
+        const long rowk = long(k0) * N1, rowq = long(r0) * N1;
+        if (k0 == row_b) __syncthreads();  // the zeroed buffers
+        // the first step's operands: all GT points of the window
+        for (int e = tid; e < GT * nc * P; e += NT) {
+            const int s = e / (nc * P), m = e - s * (nc * P), c = m / P, p = m - c * P;
+            int al, be;
+            pair_of(p, nb, 1, al, be);
+            const double2* u = a.U + (rowq + (q1f + s) % N1) * nb * nb;
+            ring[s * sz.ring + c * Pp + p] = cmul(cconj(u[al * nb + nv + c]), u[be * nb + nv + c]);
+        }
+#pragma unroll
+        for (int t = 0; t < NA; ++t)
+            if (ad[t] >= 0) {
+                const double2* u = a.U + rowk * nb * nb;
+                bufA[ad[t]] = cmul(u[a1[t]], cconj(u[a2[t]]));
+            }
+#pragma unroll
+        for (int t = 0; t < NR; ++t)
+            if (rd[t] >= 0)
+                bufR[rd[t]] = 1.0 / (a.eps[rowk * nb + rv[t]] - a.eps[(rowq + (q1f + rs[t]) % N1) * nb + nv + rc[t]]);
+        __syncthreads();
+        // The operands of step k1 + 1 are formed at the start of step k1, from
+        // loads issued one step earlier: the loads of step k1 + 2 are in flight
+        // while step k1 multiplies.
+        int oB[UPW];  // this lane's point in the ring
+#pragma unroll
+        for (int u = 0; u < UPW; ++u) oB[u] = (4 * uq[u] + g) * sz.ring + 16 * ut[u] + i;
+        double2 xa[NA], ya[NA], xb[NB], yb[NB];
+        double ev[NR], ec[NR];
+        int lk = 1, newc = (q1f + GT) % N1;  // step to load next, and the column that enters the window with it
+        int qc[NR];                          // column of each reciprocal's point in that step
+#pragma unroll
+        for (int t = 0; t < NR; ++t) qc[t] = (q1f + rs[t] + 1) % N1;
+        auto load = [&]() {
+            if (lk >= N1) return;
+            const double2* uk = a.U + (rowk + lk) * nb * nb;
+            const double2* un = a.U + (rowq + newc) * nb * nb;
+            const double* ek = a.eps + (rowk + lk) * nb;
+            const double* eq = a.eps + rowq * nb + nv;
+#pragma unroll
+            for (int t = 0; t < NA; ++t)
+                if (ad[t] >= 0) {
+                    xa[t] = uk[unsigned(a1[t])];
+                    ya[t] = uk[unsigned(a2[t])];
+                }
+#pragma unroll
+            for (int t = 0; t < NB; ++t)
+                if (bd[t] >= 0) {
+                    xb[t] = un[unsigned(b1[t])];
+                    yb[t] = un[unsigned(b2[t])];
+                }
+#pragma unroll
+            for (int t = 0; t < NR; ++t)
+                if (rd[t] >= 0) {
+                    ev[t] = ek[unsigned(rv[t])];
+                    ec[t] = eq[unsigned(qc[t] * nb + rc[t])];
+                    if (++qc[t] >= N1) qc[t] = 0;
+                }
+            ++lk;
+            if (++newc >= N1) newc = 0;
+        };
+        load();
+        int slot = GT * sz.ring;  // the ring slot behind the window, free during a step
+        for (int k1 = 0; k1 < N1; ++k1) {
+            const int par = k1 & 1;
+            if (k1 + 1 < N1) {
+                double2* An = bufA + (par ^ 1) * sz.A;
+                double2* Bn = ring + slot;
+#pragma unroll
+                for (int t = 0; t < NA; ++t)
+                    if (ad[t] >= 0) An[ad[t]] = cmul(xa[t], cconj(ya[t]));
+#pragma unroll
+                for (int t = 0; t < NB; ++t)
+                    if (bd[t] >= 0) Bn[bd[t]] = cmul(cconj(xb[t]), yb[t]);
+                double* Rn = bufR + (par ^ 1) * sz.r;
+#pragma unroll
+                for (int t = 0; t < NR; ++t)
+                    if (rd[t] >= 0) Rn[rd[t]] = 1.0 / (ev[t] - ec[t]);
+                slot += sz.ring;
+                if (slot >= ring_end) slot = 0;
+                load();
+            }
+            const double2* A = bufA + par * sz.A;
+            const double* R = bufR + par * sz.r;
+#pragma unroll
+            for (int u = 0; u < UPW; ++u) {
+                double2 x[CV], b[4 * CC];
+                double r[CC][CV];
+#pragma unroll
+                for (int vc = 0; vc < CV; ++vc) x[vc] = A[oA[u] + 4 * vc * Pp];
+#pragma unroll
+                for (int cc = 0; cc < CC; ++cc)
+#pragma unroll
+                    for (int vc = 0; vc < CV; ++vc) r[cc][vc] = R[oR[u] + cc * 16 * CV + 4 * vc];
+#pragma unroll
+                for (int c = 0; c < 4 * CC; ++c) b[c] = ring[oB[u] + oc[c]];
+                dbl4 sr[CC], si[CC];
+#pragma unroll
+                for (int cc = 0; cc < CC; ++cc) {
+                    sr[cc] = si[cc] = dbl4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                    for (int vc = 0; vc < CV; ++vc) {
+                        sr[cc] = __builtin_amdgcn_mfma_f64_16x16x4f64(r[cc][vc], x[vc].x, sr[cc], 0, 0, 0);
+                        si[cc] = __builtin_amdgcn_mfma_f64_16x16x4f64(r[cc][vc], x[vc].y, si[cc], 0, 0, 0);
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < 4 * CC; ++c) {
+                    const double re = sr[c / 4][c % 4], im = si[c / 4][c % 4];
+                    acc[u].x = fma(re, b[c].x, fma(-im, b[c].y, acc[u].x));
+                    acc[u].y = fma(re, b[c].y, fma(im, b[c].x, acc[u].y));
+                }
+                oB[u] += sz.ring;
+                if (oB[u] >= ring_end) oB[u] -= ring_end;
+            }
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < UPW; ++u) {
+        const int p = 16 * ut[u] + i, q1 = q1f + 4 * uq[u] + g;
+        if (!uok[u] || p >= P || q1 >= N1) continue;
+        const int q = q0 * N1 + q1;
+        if (a.KS > 1) {
+            *lindhard_part(a, ks, p, q) = acc[u];
+            continue;
+        }
+        int al, be;
+        pair_of(p, nb, 1, al, be);
+        const double2 x = cscale(acc[u], a.inv_nk);
+        a.X[long(al * nb + be) * a.Nk + q] = x;
+        if (al != be) a.X[long(be * nb + al) * a.Nk + q] = cconj(x);
+    }
+}
+
+constexpr int kLindSumQ = 16;  // points per work-group of the sum
+
+// X from the parts of the k range; a work-group reads every part of its points
+// before it writes (the parts lie in planes of X)
+__global__ void __launch_bounds__(256) lindhard_sum_kernel(LindhardMfmaArgs a)
+{
+    extern __shared__ double2 lds[];  // [P][kLindSumQ]
+    const int qa = blockIdx.x * kLindSumQ;
+    for (int e = threadIdx.x; e < a.P * kLindSumQ; e += 256) {
+        const int p = e / kLindSumQ, q = qa + e - p * kLindSumQ;
+        if (q >= a.Nk) continue;
+        double2 x = make_double2(0.0, 0.0);
+        for (int ks = 0; ks < a.KS; ++ks) x = cadd(x, *lindhard_part(a, ks, p, q));
+        lds[e] = cscale(x, a.inv_nk);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < a.P * kLindSumQ; e += 256) {
+        const int p = e / kLindSumQ, q = qa + e - p * kLindSumQ;
+        if (q >= a.Nk) continue;
+        int al, be;
+        pair_of(p, a.nb, 1, al, be);
+        a.X[long(al * a.nb + be) * a.Nk + q] = lds[e];
+        if (al != be) a.X[long(be * a.nb + al) * a.Nk + q] = cconj(lds[e]);
+    }
+}
+
+constexpr int kLindMaxUPW = 3;
+
+// The shape of the matrix-core form, and whether it is used.  Among the window
+// lengths GT that fit, and 1 to 3 parts of the k range, the one with the least
+// estimated time: rounds of resident work-groups x steps x the longer of a
+// step's FP64 issue time on a SIMD and its latency.
+//
+// The vector form is left the shapes it does better: two bands, where 3 of 16
+// columns would be used, and, where it fills the chip with four q per lane
+// (TQ = 4) or enough waves, those with more than one quadruple to pad.  us,
+// vector and matrix form: 3 bands, 1 filled, 40 x 40: 980, 487 (120 x 120: 6055,
+// 10315); 6, 3, 96 x 96: 9842, 7218; 8, 4, 48 x 48: 3003, 1235, 90 x 90: 22890,
+// 13998; 8, 7, 48 x 48: 2421, 1427 (96 x 96: 13263, 28374); 10, 5, 48 x 48: 3582,
+// 3672; 12, 6, 40 x 40: 3335, 2896; 14, 7, 30 x 30: 1569, 1352 (48 x 48: 6902, 10052).
+bool lindhard_mfma_shape(const LindhardPlan& p, LindhardMfmaArgs& best)
+{
+    const int nb = p.nb, nv = p.nv, nc = p.nc, N0 = p.N0, N1 = p.N1;
+    if (nv < 1 || nc < 1 || nb < 3) return false;
+    const int P = nb * (nb + 1) / 2, T = (P + 15) / 16, CV = (nv + 3) / 4, CC = (nc + 3) / 4;
+    const bool small = p.TQ == 1;
+    if (nb <= 4) {
+        if (!small || long(p.blocks) * p.W >= 1024) return false;
+    } else if (nb <= 8) {
+        if (!(CV == 1 && CC == 1) && (!small || (nb == 8 && nv == 1))) return false;
+    } else if (!small || nb <= 10) {
+        return false;
+    }
+    const int nt = lind_threads(CV, CC), W = nt / 64;
+    double best_cost = 1e300;
+    for (int GT = 4; GT <= 32; GT += 4) {
+        const LindhardMfmaLds sz(nv, nc, T, GT);
+        const size_t lds = size_t(sz.elems(GT)) * sizeof(double2);
+        const int units = (GT / 4) * T, upw = (units + W - 1) / W;
+        if (lds > 160 * 1024 || upw > kLindMaxUPW || GT * nc * nv > 2 * nt) continue;
+        const int per_cu = std::max(1, std::min(int(160 * 1024 / lds), 12 / W));
+        const int blocks = N0 * ((N1 + GT - 1) / GT);
+        for (int KS = 1; KS <= 3; ++KS) {
+            if (KS > 1 && N0 < 4 * KS) continue;
+            const long n = long(blocks) * KS;
+            const long rounds = (n + 256L * per_cu - 1) / (256L * per_cu);
+            const double resident = std::min<double>(per_cu, double((n + 255) / 256));  // work-groups per CU
+            const double unit = 128.0 * CV * CC + 64.0 * CC + 60.0;             // issue cycles of one unit
+            const double build = 4.0 * (14.0 * P * nb + 30.0 * GT * nc * nv) / nt;  // per wave
+            const double wave = upw * unit + build;
+            const double step = std::max(600.0 + wave, resident * W / 4 * wave);
+            const double cost = double(rounds) * ((N0 + KS - 1) / KS) * (N1 + 3) * step;
+            if (cost < best_cost) {
+                best_cost = cost;
+                best.GT = GT;
+                best.KS = KS;
+            }
+        }
+    }
+    if (best_cost >= 1e300) return false;
+    best.nb = nb;
+    best.nv = nv;
+    best.nc = nc;
+    best.N0 = N0;
+    best.N1 = N1;
+    best.Nk = N0 * N1;
+    best.P = P;
+    best.T = T;
+    best.nqb_row = (N1 + best.GT - 1) / best.GT;
+    best.inv_nk = 1.0 / double(best.Nk);
+    return true;
+}
+
+// false: not launched.  More than 64 KB of LDS needs the kernel's limit raised,
+// which does not reach a launch that is being captured: a first call under
+// capture is left to the vector form.
+template <int CV, int CC, int UPW>
+bool launch_mfma_one(const LindhardMfmaArgs& a, hipStream_t s)
+{
+    const size_t lds = size_t(LindhardMfmaLds(a.nv, a.nc, a.T, a.GT).elems(a.GT)) * sizeof(double2);
+    auto kern = &lindhard_mfma_kernel<CV, CC, UPW>;
+    static std::atomic<bool> raised{false};  // calls may come from several host threads
+    if (lds > 64 * 1024 && !raised.load()) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (s) EDUS_HIP_CHECK(hipStreamIsCapturing(s, &st));
+        if (st != hipStreamCaptureStatusNone) return false;
+        EDUS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        raised.store(true);
+    }
+    hipLaunchKernelGGL(kern, dim3(a.N0 * a.nqb_row * a.KS), dim3(lind_threads(CV, CC)), lds, s, a);
+    return true;
+}
+
+template <int CV, int CC>
+bool launch_mfma_upw(const LindhardMfmaArgs& a, hipStream_t s)
+{
+    const int W = lind_threads(CV, CC) / 64;
+    switch (((a.GT / 4) * a.T + W - 1) / W) {
+        case 1: return launch_mfma_one<CV, CC, 1>(a, s);
+        case 2: return launch_mfma_one<CV, CC, 2>(a, s);
+        default: return launch_mfma_one<CV, CC, kLindMaxUPW>(a, s);
+    }
+}
+
+bool launch_lindhard_mfma(const LindhardMfmaArgs& a, hipStream_t s)
+{
+    bool done = false;
+    switch ((a.nv + 3) / 4 * 8 + (a.nc + 3) / 4) {
+#define EDUS_CVCC(cv, cc) \
+    case cv * 8 + cc: done = launch_mfma_upw<cv, cc>(a, s); break;
+        EDUS_CVCC(1, 1) EDUS_CVCC(1, 2) EDUS_CVCC(1, 3) EDUS_CVCC(1, 4) EDUS_CVCC(2, 1) EDUS_CVCC(2, 2)
+        EDUS_CVCC(2, 3) EDUS_CVCC(3, 1) EDUS_CVCC(3, 2) EDUS_CVCC(4, 1)
+#undef EDUS_CVCC
+        default: break;
+    }
+    if (!done) return false;
+    if (a.KS > 1)
+        hipLaunchKernelGGL(lindhard_sum_kernel, dim3((a.Nk + kLindSumQ - 1) / kLindSumQ), dim3(256),
+                           size_t(a.P) * kLindSumQ * sizeof(double2), s, a);
+    EDUS_HIP_CHECK(hipGetLastError());
+    return true;
 }
 
 // waves per q for L element pairs (fractional when several q share a wave)
@@ -436,6 +871,14 @@ void launch_lindhard(const LindhardPlan& p, const double2* U, const double* eps,
         hipLaunchKernelGGL(lindhard_zero_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, X, n);
         EDUS_HIP_CHECK(hipGetLastError());
         return;
+    }
+    LindhardMfmaArgs m{};
+    if (lindhard_mfma_shape(p, m)) {
+        m.U = U;
+        m.eps = eps;
+        m.X = X;
+        m.work = work;
+        if (launch_lindhard_mfma(m, s)) return;
     }
     double2* Uv = work;
     double2* Uc = work + size_t(p.Nk) * p.nv * p.nb;
