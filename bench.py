@@ -28,7 +28,8 @@ HBM_PEAK_GBS = 8000.0
 
 def kernel_bytes(cls: str, npl: int, nk: int, nb: int, n_e: int, solver: str = "RK", order: int = 4,
                  coulomb: bool = False, peierls: bool = False, f32_fields: bool = False,
-                 tri_fields: bool = False, hf_fused: bool = False) -> float:
+                 tri_fields: bool = False, hf_fused: bool = False, carried_sum: bool = True,
+                 derivatives: int = 1) -> float:
     """Algorithmic HBM bytes per launch: one array of npl planes is
     S = npl*nk*16 B.  grad_col reads rho, writes G (2S); grad_row reads rho
     and G, writes D (3S); grad_fused (both axes in one pass per plane) reads
@@ -55,6 +56,10 @@ def kernel_bytes(cls: str, npl: int, nk: int, nb: int, n_e: int, solver: str = "
     comm = (5.5 + n_e + sig) if solver == "RK" else (4 + n_e + order + sig)
     if peierls:
         comm -= 1 + n_e
+    else:
+        comm += derivatives - 1
+    if solver == "RK" and not carried_sum:
+        comm -= 0.25
     field = 1.0  # bytes of H0 and of each xi, in arrays
     if f32_fields:
         field *= 0.5
@@ -62,7 +67,7 @@ def kernel_bytes(cls: str, npl: int, nk: int, nb: int, n_e: int, solver: str = "
         field *= (nb + 1) / (2.0 * nb)
     if not peierls:
         comm -= (1.0 - field) * (1 + n_e)
-    return {"grad_col": 2 * s, "grad_row": (4 if (coulomb and hf_fused) else 3) * s, "grad_fused": 2 * s, "kgrad": 2 * s, "comm": comm * s,
+    return {"grad_col": 2 * s, "grad_row": (4 if (coulomb and hf_fused) else 3) * s, "grad_fused": 2 * s, "kgrad": 2 * s, "comm": comm * s, "grad_axes": 4 * s,
             "hf_row": 2 * s,
             "hf_col": 2.5 * s, "peierls_col": (2 + n_e) * s,
             "peierls_row": 2 * s, "hf_plane": 3.5 * s, "peierls_plane": (2 + n_e) * s}.get(cls, 0.0)
@@ -107,18 +112,18 @@ def cpu_baseline(params: dict, steps: int, integ: str, bytes_per_kstep: float = 
 
 
 def measured_traffic(cls: str, workload: str, layout: str, precision: str, gradient: str = "R",
-                     gauge: str = "length", fields: str = "full"):
+                     gauge: str = "length", fields: str = "full", derivatives: str = "1"):
     """HBM bytes per launch of a kernel class from the committed rocprofv3
     counter summaries under profiles/ (FETCH_SIZE and WRITE_SIZE runs scaled
     by the copy-kernel calibration); None when no summary covers the case.
-    A summary without a gradient=, gauge= or fields= key covers the defaults
-    (the spectral gradient, the length gauge, H0 and xi read from every
-    element) only."""
+    A summary without a gradient=, gauge=, fields= or derivatives= key covers
+    the defaults (the spectral gradient, the length gauge, H0 and xi read from
+    every element, one array of E.grad rho) only."""
     import glob
 
     want = {"class": cls, "workload": workload, "layout": layout, "precision": precision,
-            "gradient": gradient, "gauge": gauge, "fields": fields}
-    default = {"gradient": "R", "gauge": "length", "fields": "full"}
+            "gradient": gradient, "gauge": gauge, "fields": fields, "derivatives": derivatives}
+    default = {"gradient": "R", "gauge": "length", "fields": "full", "derivatives": "1"}
     for path in sorted(glob.glob(os.path.join(ROOT, "profiles", "*.txt"))):
         with open(path) as f:
             for line in f:
@@ -250,7 +255,7 @@ def main():
     sim.steps(args.steps)
     eng.synchronize()
     elapsed_direct = time.perf_counter() - t1
-    classes = ["grad_col", "grad_row", "grad_fused", "kgrad", "comm", "hf_row", "hf_col", "hf_plane", "peierls_col",
+    classes = ["grad_col", "grad_row", "grad_axes", "grad_fused", "kgrad", "comm", "hf_row", "hf_col", "hf_plane", "peierls_col",
                "peierls_row", "peierls_plane"]
     times = {c: eng.timing_get(c) for c in classes}
     eng.timing_enable(False)
@@ -266,15 +271,18 @@ def main():
     tun = eng.get_tuning()
     tri = bool(tun.tri_fields)  # H0 and xi read from their upper triangles
     hf = coul and bool(tun.hf_fused) and tun.fft_family[1] == 1  # exchange row pass from the gradient's
-    kb = {c: kernel_bytes(c, npl, nk, nb, n_e, solver, order, coul, bool(args.peierls), f32, tri, hf)
-          for c in classes}
+    # a field along one grid axis gives one array of derivatives either way
+    nd = 0 if args.gradient_space == "k" and not times["kgrad"][1] else 2 if times["grad_axes"][1] else 1
+    kb = {c: kernel_bytes(c, npl, nk, nb, n_e, solver, order, coul, bool(args.peierls), f32, tri, hf,
+                          args.precision == "mixed", nd) for c in classes}
     dom = max(classes, key=lambda c: times[c][0])
     ms, cnt = times[dom]
     avg_s = ms / 1e3 / max(cnt, 1)
     byts = kb[dom]
     achieved = byts / avg_s / 1e9
     traffic, traffic_src = measured_traffic(dom, args.workload, args.layout, args.precision, args.gradient_space,
-                                            "peierls" if args.peierls else "length", "tri" if tri else "full")
+                                            "peierls" if args.peierls else "length", "tri" if tri else "full",
+                                            "1" if args.peierls else str(nd))
     roofline = {"bound": "hbm", "kernel": dom, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "traffic_source": traffic_src,
                 "bytes_per_launch": byts,

@@ -29,6 +29,9 @@ void launch_comm(int nb, int layout, int kind, int tile, const CommArgs& args, h
     }
     if (args.tri && (layout != kFull || args.sigma || args.hsum || kind == kCommScalar))
         throw std::runtime_error("upper-triangle H0 and xi: FULL layout without exchange, MFMA engines only");
+    if (args.nst > 0 && (args.up.ab_order > 0 || args.up.out1 == args.rho || args.up.out2 == args.rho))
+        throw std::runtime_error("the stencil reads the stage input at other k-points: it must not be overwritten");
+    if (args.D2 && !args.D) throw std::runtime_error("a second derivative array needs the first");
     if (args.hsum && !args.hart) throw std::runtime_error("the Hartree shift needs V with the plane sums");
     if (kind == kCommMfma32 && args.H0f) {
         if (args.sigma) throw std::runtime_error("FP32 H0 with exchange: H0 holds -Sigma[rho0] and stays FP64");

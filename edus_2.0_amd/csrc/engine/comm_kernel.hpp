@@ -240,22 +240,88 @@ __device__ inline void mfma_commutator32(const double2* sH, const double2* sR, i
 
 // AB: the stage is an Adams-Bashforth step (its history is prefetched, so the
 // register budget of the other stages does not carry four history arrays).
-// x1 += g1 (rho - x2) for a thread's elements, rho read from the tile
+// x1 <- rho + g1 (x1 - rho), or with carried x1 <- x1 + g1 (rho - x2), for a
+// thread's elements, rho read from the tile
 template <int PER>
-__device__ inline void fold_g1(double g1, const double2* sR, const int (&slot_of)[PER], const bool (&ok)[PER],
-                               const double2 (&x2)[PER], double2 (&x1)[PER])
+__device__ inline void fold_g1(double g1, bool carried, const double2* sR, const int (&slot_of)[PER],
+                               const bool (&ok)[PER], const double2 (&x2)[PER], double2 (&x1)[PER])
 {
 #pragma unroll
     for (int j = 0; j < PER; ++j)
         if (ok[j]) {
             const double2 r = sR[slot_of[j]];
-            x1[j].x += g1 * (r.x - x2[j].x);
-            x1[j].y += g1 * (r.y - x2[j].y);
+            if (carried) {
+                x1[j].x += g1 * (r.x - x2[j].x);
+                x1[j].y += g1 * (r.y - x2[j].y);
+            } else {
+                x1[j].x = r.x + g1 * (x1[j].x - r.x);
+                x1[j].y = r.y + g1 * (x1[j].y - r.y);
+            }
         }
 }
 
-template <int NB, int LAYOUT, int KIND, int TILE, bool AB, bool TRI>
-__global__ void __launch_bounds__((comm_threads<KIND, TILE>())) comm_kernel(CommArgs a)
+// D at a thread's elements from the finite-difference stencil: sum_b w_b (b.E)
+// rho(k + b), in the order and arithmetic of kgrad_kernel.  Every element of a
+// thread has the same k-point, so a tap's offset is formed once; kTaps taps'
+// loads are issued before the first is used.  Neighbouring tiles run side by
+// side in one XCD, so the taps come from its L2 mostly.
+template <int PER>
+__device__ inline void stencil_taps(const CommArgs& a, const double Ev[3], int k, const long (&off)[PER],
+                                    const bool (&ok)[PER], double2 (&dv)[PER])
+{
+    constexpr int kTaps = PER <= 2 ? 6 : 3;
+    const int i0 = k / a.N1, i1 = k - (k / a.N1) * a.N1;
+    for (int b0 = 0; b0 < a.nst; b0 += kTaps) {
+        double2 v[kTaps][PER];
+        double c[kTaps];
+#pragma unroll
+        for (int t = 0; t < kTaps; ++t) {
+            if (b0 + t >= a.nst) break;
+            const KStencilPoint& q = a.kst[b0 + t];
+            int j0 = i0 + q.m0, j1 = i1 + q.m1;
+            if (j0 < 0) j0 += a.N0;
+            if (j0 >= a.N0) j0 -= a.N0;
+            if (j1 < 0) j1 += a.N1;
+            if (j1 >= a.N1) j1 -= a.N1;
+            const double bdotu = q.b[0] * Ev[0] + q.b[1] * Ev[1] + q.b[2] * Ev[2];
+            c[t] = q.w * bdotu;
+            const long d = long(j0) * a.N1 + j1 - k;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                v[t][j] = make_double2(0., 0.);
+                if (ok[j]) v[t][j] = a.rho[off[j] + d];
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < kTaps; ++t) {
+            if (b0 + t >= a.nst) break;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                dv[j].x += c[t] * v[t][j].x;
+                dv[j].y += c[t] * v[t][j].y;
+            }
+        }
+    }
+}
+
+// EXT: the derivative is not one array: a second one (kExtD2, CommArgs::D2) or
+// the finite-difference stencil (kExtStencil, CommArgs::kst; RK4 only: an
+// Adams-Bashforth step updates the state it reads); separate instantiations, so
+// that the other kernels keep their registers
+enum CommExt { kExtNone = 0, kExtD2 = 1, kExtStencil = 2 };
+
+// Tile 2 with upper-triangle fields keeps to 128 registers, two work-groups per
+// CU (14 bands, FP32 engine: 136 without the limit, one work-group per CU and
+// 75 us at 120 x 120 instead of 48); where the limit would spill it is left off.
+template <int NB, int KIND, int TILE, bool AB, bool TRI, int EXT>
+constexpr int comm_min_waves()
+{
+    return TILE == 2 && TRI && !AB && EXT != kExtStencil && NB <= 14 ? 4 : 1;
+}
+
+template <int NB, int LAYOUT, int KIND, int TILE, bool AB, bool TRI, int EXT>
+__global__ void __launch_bounds__((comm_threads<KIND, TILE>()),
+                                  (comm_min_waves<NB, KIND, TILE, AB, TRI, EXT>())) comm_kernel(CommArgs a)
 {
     static_assert(!TRI || (LAYOUT == kFull && KIND != kCommScalar), "upper-triangle fields: FULL, MFMA engines");
     constexpr int NT = comm_threads<KIND, TILE>();
@@ -514,6 +580,14 @@ __global__ void __launch_bounds__((comm_threads<KIND, TILE>())) comm_kernel(Comm
         for (int j = 0; j < PER; ++j)
             if (ok[j]) dv[j] = a.D[off[j]];
     }
+    double2 dv2[EXT == kExtD2 ? PER : 1];
+    if constexpr (EXT == kExtD2) {
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            dv2[j] = zero;
+            if (ok[j]) dv2[j] = a.D2[off[j]];
+        }
+    }
     if (ld_x1) {
 #pragma unroll
         for (int j = 0; j < PER; ++j)
@@ -533,6 +607,8 @@ __global__ void __launch_bounds__((comm_threads<KIND, TILE>())) comm_kernel(Comm
                     if (ok[j]) ex[i - 1][j] = u.hist[i][off[j]];
             }
     }
+    if constexpr (EXT == kExtStencil)  // NT is a multiple of TK: a thread's elements share their k-point
+        stencil_taps<PER>(a, Ev, k0 + int(threadIdx.x) % TK, off, ok, dv);
     if (u.mon) {
         // Trace and Hermiticity of the stage input (the state the step starts
         // from: RK4 stage 1, every AB step) over the tile's TK k-points, read
@@ -596,7 +672,7 @@ __global__ void __launch_bounds__((comm_threads<KIND, TILE>())) comm_kernel(Comm
             else
                 mfma_commutator32<NB, LAYOUT, PS>(sH, sR, kk, lane, tri, cre[w], cim[w]);
         }
-        if (!ab && u.g1 != 0.0) fold_g1(u.g1, sR, slot_of, ok, ex[0], x1v);  // rho before the products replace it
+        if (!ab && u.g1 != 0.0) fold_g1(u.g1, u.g1_carried != 0, sR, slot_of, ok, ex[0], x1v);  // rho before the products replace it
         __syncthreads();
         const int i = lane & 15, q = lane >> 4;
 #pragma unroll
@@ -617,7 +693,7 @@ __global__ void __launch_bounds__((comm_threads<KIND, TILE>())) comm_kernel(Comm
     }
 
     if constexpr (KIND == kCommScalar && !AB)  // rho stays in the tile
-        if (u.g1 != 0.0) fold_g1(u.g1, sR, slot_of, ok, ex[0], x1v);
+        if (u.g1 != 0.0) fold_g1(u.g1, u.g1_carried != 0, sR, slot_of, ok, ex[0], x1v);
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
         if (!ok[j]) continue;
@@ -645,6 +721,7 @@ __global__ void __launch_bounds__((comm_threads<KIND, TILE>())) comm_kernel(Comm
             acc = sR[p * PS + kk];
         }
         const long og = off[j];
+        if constexpr (EXT == kExtD2) dv[j] = cadd(dv[j], dv2[j]);
         // f = D - i * [H, rho]
         const double2 f = make_double2(dv[j].x + acc.y, dv[j].y - acc.x);
 
@@ -686,12 +763,13 @@ __global__ void __launch_bounds__((comm_threads<KIND, TILE>())) comm_kernel(Comm
     }
 }
 
-template <int NB, int LAYOUT, int KIND, int TILE, bool AB, bool TRI>
+template <int NB, int LAYOUT, int KIND, int TILE, bool AB, bool TRI, int EXT>
 void launch_one(const CommArgs& a, hipStream_t s)
 {
     constexpr int TK = tile_k<NB, LAYOUT, KIND, TILE>();
     constexpr size_t lds = comm_lds_bytes<NB, LAYOUT, KIND, TILE, TRI>();
-    auto kern = &comm_kernel<NB, LAYOUT, KIND, TILE, AB, TRI>;
+    auto kern = &comm_kernel<NB, LAYOUT, KIND, TILE, AB, TRI, EXT>;
+    static_assert(comm_threads<KIND, TILE>() % TK == 0, "one k-point per thread");
     static std::once_flag raised;  // contexts may be created from several host threads
     std::call_once(raised, [&] {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -705,10 +783,18 @@ void launch_one(const CommArgs& a, hipStream_t s)
 template <int NB, int LAYOUT, int KIND, int TILE, bool TRI>
 void launch_ab(const CommArgs& a, hipStream_t s)
 {
-    if (a.up.ab_order > 0)
-        launch_one<NB, LAYOUT, KIND, TILE, true, TRI>(a, s);
-    else
-        launch_one<NB, LAYOUT, KIND, TILE, false, TRI>(a, s);
+    if (a.up.ab_order > 0) {
+        if (a.D2)
+            launch_one<NB, LAYOUT, KIND, TILE, true, TRI, kExtD2>(a, s);
+        else
+            launch_one<NB, LAYOUT, KIND, TILE, true, TRI, kExtNone>(a, s);
+    } else if (a.nst > 0) {
+        launch_one<NB, LAYOUT, KIND, TILE, false, TRI, kExtStencil>(a, s);
+    } else if (a.D2) {
+        launch_one<NB, LAYOUT, KIND, TILE, false, TRI, kExtD2>(a, s);
+    } else {
+        launch_one<NB, LAYOUT, KIND, TILE, false, TRI, kExtNone>(a, s);
+    }
 }
 
 template <int NB, int LAYOUT, int KIND, int TILE>

@@ -104,9 +104,9 @@ std::map<std::tuple<int, int, int, int>, FFTChoice>& tuned_shapes()
 }
 
 // commutator engine and tile per (nb, layout, k-points of all instances,
-// precision, kept engine, exchange, upper-triangle fields): the last two
-// change the bytes per launch
-using CommKey = std::tuple<int, int, int, int, int, int, int>;
+// precision, kept engine, exchange, upper-triangle fields, form of the
+// derivative): the last three change the bytes per launch
+using CommKey = std::tuple<int, int, int, int, int, int, int, int>;
 std::map<CommKey, std::tuple<int, int, int>>& tuned_comm()
 {
     static std::map<CommKey, std::tuple<int, int, int>> m;
@@ -686,7 +686,8 @@ void Engine::autotune()
     // mixed precision the FP32 matrix cores; tiles give identical results.
     // The Adams-Bashforth kernel (history prefetched, more registers) gets a
     // tile of its own.
-    const CommKey ckey = std::make_tuple(nb, layout, Nk * B, prec, force_kind, int(coulomb), int(tri));
+    const CommKey ckey = std::make_tuple(nb, layout, Nk * B, prec, force_kind, int(coulomb), int(tri),
+                                         kgrad ? (stencil_fused() ? 2 : 0) : int(axes_together()));
     auto cit = tuned_comm().find(ckey);
     if (cit != tuned_comm().end()) {
         comm_kind = std::get<0>(cit->second);
@@ -708,9 +709,17 @@ void Engine::autotune()
         HIP_CHECK(hipEventCreate(&e0));
         HIP_CHECK(hipEventCreate(&e1));
         auto time_of = [&](int kind, int tile, const CommArgs& c) {
-            launch_comm(nb, layout, kind, tile, c, s);  // warm-up
+            // with the stage's set, and for RK4 the other stages': one array read
+            // and written beside the operands
+            CommArgs lite = c;
+            if (!c.up.ab_order) lite.up.out1 = nullptr;
+            auto step = [&] {
+                for (int r = 0; r < 4; ++r) launch_comm(nb, layout, kind, tile, r == 2 ? c : lite, s);
+            };
+            step();  // warm-up
             HIP_CHECK(hipEventRecord(e0, s));
-            for (int r = 0; r < 3; ++r) launch_comm(nb, layout, kind, tile, c, s);
+            step();
+            step();
             HIP_CHECK(hipEventRecord(e1, s));
             HIP_CHECK(hipEventSynchronize(e1));
             float ms = 0.f;
@@ -726,6 +735,11 @@ void Engine::autotune()
         auto ab_args = [&](int kind) {
             CommArgs cab = tuning_stage_args(kind);
             cab.up = StageUpdate{};
+            if (cab.nst > 0) {  // an Adams-Bashforth step updates the state in place: a stencil pass of its own
+                cab.nst = 0;
+                cab.D = D;
+            }
+            if (cab.D2) cab.D2 = f;
             cab.up.ab_order = 4;
             cab.up.y = aux;
             cab.up.out_f = G;
@@ -777,14 +791,15 @@ void Engine::autotune()
             const double cg[2] = {1e-3, 1e-3};
             CommArgs c = tuning_stage_args(comm_kind);
             float best[2] = {1e30f, 1e30f};
-            for (int trial = 0; trial < 2; ++trial)
+            for (int trial = 0; trial < 3; ++trial)
                 for (int f = 0; f < 2; ++f) {
                     grad_fused = f == 1;
-                    c.D = gradient(c.rho, cg, nullptr, true, true);  // warm-up
+                    c.D = c.D2 = nullptr;
+                    derivative_terms(c, cg, nullptr, nullptr, nullptr, true, true);  // warm-up
                     launch_comm(nb, layout, comm_kind, comm_tile, c, s);
                     HIP_CHECK(hipEventRecord(e0, s));
-                    for (int r = 0; r < 4; ++r) {
-                        gradient(c.rho, cg, nullptr, true, true);
+                    for (int r = 0; r < 8; ++r) {
+                        derivative_terms(c, cg, nullptr, nullptr, nullptr, true, true);
                         launch_comm(nb, layout, comm_kind, comm_tile, c, s);
                     }
                     HIP_CHECK(hipEventRecord(e1, s));
@@ -796,7 +811,7 @@ void Engine::autotune()
             (void)hipEventDestroy(e0);
             (void)hipEventDestroy(e1);
             HIP_CHECK(hipGetLastError());
-            grad_fused = best[1] < best[0];
+            grad_fused = best[1] < 0.98f * best[0];  // the two passes unless the other form is clearly faster
             tuned_grad()[gkey] = grad_fused;
         }
     }
@@ -833,10 +848,18 @@ CommArgs Engine::tuning_stage_args(int kind) const
             break;
         }
     field_args(c, use_xi, kind);
-    c.D = D;
+    if (kgrad && stencil_fused()) {
+        c.kst = kst_dev;
+        c.nst = int(kst.size());
+        c.N0 = N0;
+        c.N1 = N1;
+    } else {
+        c.D = D;
+        if (axes_together()) c.D2 = G;
+    }
     c.up.x1 = acc;
     c.up.out1 = acc;
-    c.up.g1 = 2. / 3.;
+    c.up.g1 = 1. / 3.;
     c.up.x2 = y;
     c.up.out2 = f;
     return c;
@@ -865,6 +888,7 @@ void Engine::prime_launch_attributes()
     c.B = B;
     c.H0 = H0;
     c.H0f = H0f ? H0f : reinterpret_cast<const float2*>(H0);  // not launched
+    c.rho = aux;
     for (int t = 0; t < (tri_ok ? 2 : 1); ++t)  // both H0 / xi storages (separate kernels)
         for (int ab = 0; ab < 2; ++ab) {
             c.up = StageUpdate{};
@@ -872,8 +896,13 @@ void Engine::prime_launch_attributes()
             for (int kind : {comm_kind, comm_kind64}) {
                 c.tri = t == 1 && kind != kCommScalar;
                 if (t == 1 && !c.tri) continue;
-                for (int tile : {0, 1, 2})
-                    if (tile == 0 || kind != kCommScalar) launch_comm(nb, layout, kind, tile, c, s);
+                for (int form = 0; form < 3; ++form) {  // one derivative array, two, the stencil
+                    c.D = c.D2 = form == 1 ? D : nullptr;
+                    c.nst = form == 2 ? 1 : 0;
+                    if (form == 2 && ab) continue;
+                    for (int tile : {0, 1, 2})
+                        if (tile == 0 || kind != kCommScalar) launch_comm(nb, layout, kind, tile, c, s);
+                }
             }
         }
     if (U) {
@@ -998,17 +1027,59 @@ void Engine::fock(const double2* in, bool row_done)
     axis_fft(1, 2, T, nullptr, T, 0.0, 1.0, nullptr, "hf_row");
 }
 
-// D = E . grad rho (as gradient) and, with exchange, T of the same input
-const double2* Engine::spectral_terms(const double2* in, const double c[2], const double* ctab, bool use0, bool use1)
+// The derivative of c.rho as the commutator takes it (c.D, c.D2 or the stencil)
+// and, with exchange, T of the same input: with the coefficients cc of the grid
+// axes (or per instance ctab) and, for the k-space gradient, the field E (E_tab)
+void Engine::derivative_terms(CommArgs& c, const double cc[2], const double* ctab, const double* E,
+                              const double* E_tab, bool use0, bool use1)
 {
+    const double2* in = c.rho;
+    if (kgrad) {
+        if (use0 || use1) {
+            if (stencil_fused() && c.up.out1 != in && c.up.out2 != in && c.up.y != in) {
+                c.kst = kst_dev;
+                c.nst = int(kst.size());
+                c.N0 = N0;
+                c.N1 = N1;
+            } else {
+                c.D = kgradient(in, E, E_tab);
+            }
+        }
+        if (coulomb) fock(in);
+        return;
+    }
     if (coulomb && plane_exchange() && ((use0 && N0 > 1) || (use1 && N1 > 1))) {  // both from one launch
-        plane_launch(in, true, c, ctab, true);
-        return D;
+        plane_launch(in, true, cc, ctab, true);
+        c.D = D;
+        return;
+    }
+    if (axes_together()) {
+        use0 = use0 && N0 > 1;
+        use1 = use1 && N1 > 1;
+        if (use0 || use1) {
+            PlaneArgs a = axes_args(N0, N1);
+            a.in = in;
+            a.out[0] = use0 ? G : nullptr;
+            a.out[1] = use1 ? D : nullptr;
+            a.P = B * npl;
+            a.tw0 = tw[0];
+            a.tw1 = tw[1];
+            for (int j = 0; j < 2; ++j) a.coef[j] = cc[j];
+            a.coef_tab = ctab;
+            a.coef_stride = 2;
+            a.ppi = npl;
+            TimedLaunch t;
+            tbegin("grad_axes", t);
+            launch_axes(a, s);
+            tend(t);
+            c.D = use1 ? D : G;
+            c.D2 = use0 && use1 ? G : nullptr;
+        }
+        return;
     }
     bool hf_row = false;  // the exchange term's forward row pass done by the gradient
-    const double2* Dp = gradient(in, c, ctab, use0, use1, coulomb && hf_fuse ? T : nullptr, &hf_row);
+    c.D = gradient(in, cc, ctab, use0, use1, coulomb && hf_fuse ? T : nullptr, &hf_row);
     if (coulomb) fock(in, hf_row);
-    return Dp;
 }
 
 void Engine::transform_to_R(const double2* in, double2* out)
@@ -1031,18 +1102,12 @@ void Engine::evaluate(const double2* in, const double E[3], const StageUpdate& u
 {
     double cg[2];
     for (int j = 0; j < 2; ++j) cg[j] = (A[0][j] * E[0] + A[1][j] * E[1] + A[2][j] * E[2]) / (j == 0 ? N0 : N1);
-    const double2* Dp;
-    if (kgrad) {
-        Dp = (cg[0] != 0.0 || cg[1] != 0.0) ? kgradient(in, E, nullptr) : nullptr;
-        if (coulomb) fock(in);
-    } else {
-        Dp = spectral_terms(in, cg, nullptr, cg[0] != 0.0, cg[1] != 0.0);
-    }
     CommArgs c{};
     c.Nk = Nk;
     c.P = npl;
     c.rho = in;
-    c.D = Dp;
+    c.up = up;
+    derivative_terms(c, cg, nullptr, E, nullptr, cg[0] != 0.0, cg[1] != 0.0);
     const bool use_xi[3] = {E[0] != 0.0, E[1] != 0.0, E[2] != 0.0};
     field_args(c, use_xi, comm_kind);
     for (int d = 0; d < 3; ++d) c.E[d] = E[d];
@@ -1058,26 +1123,48 @@ void Engine::evaluate(const double2* in, const double E[3], const StageUpdate& u
 }
 
 
-// The four stage updates of one classical RK4 step (DESolver.hpp:155-187):
-//   k1 = f(t, y);        aux = y + dt/2 k1;  acc = y + dt/6 k1     (:166-171)
-//   k2 = f(t+dt/2, aux); aux = y + dt/2 k2                         (:174-177)
-//   k3 = f(t+dt/2, aux); aux = y + dt k3;
-//                        acc += 2/3 (aux_in - y) + dt/3 k3         (:174-182)
-//   k4 = f(t+dt, aux);   y = acc + dt/6 k4                         (:184-185)
-// The reference adds dt/3 k2 to acc in stage 2; here stage 3 recovers it as
-// 2/3 (aux_in - y) = dt/3 k2 from the two arrays it reads anyway, so stage 2
-// neither reads nor writes acc (a step moves 26 plane sets instead of 28).
+// The four stage updates of one classical RK4 step (DESolver.hpp:155-187),
+//   k1 = f(t, y), k2 = f(t+dt/2, Y2), k3 = f(t+dt/2, Y3), k4 = f(t+dt, Y4),
+//   Y2 = y + dt/2 k1, Y3 = y + dt/2 k2, Y4 = y + dt k3,
+//   y  <- y + dt/6 k1 + dt/3 k2 + dt/3 k3 + dt/6 k4:
+// the reference carries the weighted sum through every stage; the stage inputs
+// hold the same terms, y + dt/6 k1 + dt/3 k2 + dt/3 k3 = (Y2 + 2 Y3 + dt k3) / 3,
+// formed in stage 3 as Y3 + (Y2 - Y3) / 3 + dt/3 k3 from two arrays it reads.
+// Stages 1 and 2 write their stage input only (a step moves 25 plane sets at
+// one field component; carrying the sum takes 28).
+//   stage 1  rho = y,   writes acc = Y2
+//   stage 2  rho = acc, writes aux = Y3
+//   stage 3  rho = aux, writes acc = the sum and, over aux, Y4
+//   stage 4  rho = Y4,  writes y
+// In mixed precision the sum is carried from stage 1 (acc = y + dt/6 k1, stage 3
+// adding dt/3 k2 as 2/3 (Y3 - y)), so that those runs keep their bits: an FP64
+// rounding there can move an FP32 one in the results.  Where the commutator
+// reads its input at other k-points too (the fused stencil) no stage may write
+// over it, and G takes the third stage array.
 // Stage 1 carries the per-step trace / Hermiticity monitor of the y the step
 // starts from (the y it writes is checked by the next step, or by
 // check_final_state).
-void Engine::rk4_stages(double dt, StageUpdate u[4]) const
+void Engine::rk4_stages(double dt, StageUpdate u[4], double2* in[4]) const
 {
     for (int i = 0; i < 4; ++i) u[i] = StageUpdate{};
-    u[0].x1 = y; u[0].out1 = acc; u[0].b1 = dt / 6.;
-    u[0].x2 = y; u[0].out2 = aux; u[0].b2 = dt / 2.;
-    u[1].x2 = y; u[1].out2 = aux; u[1].b2 = dt / 2.;
-    u[2].x1 = acc; u[2].out1 = acc; u[2].b1 = dt / 3.; u[2].g1 = 2. / 3.;
-    u[2].x2 = y; u[2].out2 = aux; u[2].b2 = dt;
+    double2* other = kgrad && stencil_fused() ? G : aux;
+    in[0] = y;
+    if (prec == EDUS_PREC_MIXED) {
+        in[1] = aux;
+        in[2] = other;
+        in[3] = aux;
+        u[0].x1 = y; u[0].out1 = acc; u[0].b1 = dt / 6.;
+        u[2].g1 = 2. / 3.; u[2].g1_carried = 1;
+    } else {
+        in[1] = acc;
+        in[2] = aux;
+        in[3] = other;
+        u[2].g1 = 1. / 3.;
+    }
+    u[0].x2 = y; u[0].out2 = in[1]; u[0].b2 = dt / 2.;
+    u[1].x2 = y; u[1].out2 = in[2]; u[1].b2 = dt / 2.;
+    u[2].x1 = acc; u[2].out1 = acc; u[2].b1 = dt / 3.;
+    u[2].x2 = y; u[2].out2 = in[3]; u[2].b2 = dt;
     u[3].x1 = acc; u[3].out1 = y; u[3].b1 = dt / 6.;
     u[0].mon = mon; u[0].nf = double(nf);
 }
@@ -1086,15 +1173,16 @@ void Engine::rk4_step(double dt, const double* E3x3, int record_order)
 {
     state_dirty = true;  // the state it writes is checked by the next step or check_final_state
     StageUpdate u[4];
-    rk4_stages(dt, u);
+    double2* in[4];
+    rk4_stages(dt, u, in);
     if (record_order > 0) {
         ensure_hist();
         u[0].out_f = hist[abidx[0]];
     }
-    evaluate(y, E3x3 + 0, u[0]);
-    evaluate(aux, E3x3 + 3, u[1]);
-    evaluate(aux, E3x3 + 3, u[2]);
-    evaluate(aux, E3x3 + 6, u[3]);
+    evaluate(in[0], E3x3 + 0, u[0]);
+    evaluate(in[1], E3x3 + 3, u[1]);
+    evaluate(in[2], E3x3 + 3, u[2]);
+    evaluate(in[3], E3x3 + 6, u[3]);
     if (record_order > 0) {  // the same rotation as ab_step
         const int tmp = abidx[record_order - 1];
         for (int i = record_order - 1; i > 0; --i) abidx[i] = abidx[i - 1];
@@ -1240,19 +1328,13 @@ void Engine::evaluate_tab(const double2* in, int ts, int j, const bool use_axis[
 {
     const size_t row = size_t(ts) * 3 + j;
     const double c0[2] = {0.0, 0.0};
-    const double2* Dp;
-    if (kgrad) {
-        Dp = (use_axis[0] || use_axis[1]) ? kgradient(in, nullptr, E_dev + row * B * 3) : nullptr;
-        if (coulomb) fock(in);
-    } else {
-        Dp = spectral_terms(in, c0, coef_dev + row * B * 2, use_axis[0], use_axis[1]);
-    }
     CommArgs c{};
     c.Nk = Nk;
     c.P = npl;
     c.B = B;
     c.rho = in;
-    c.D = Dp;
+    c.up = up;
+    derivative_terms(c, c0, coef_dev + row * B * 2, nullptr, E_dev + row * B * 3, use_axis[0], use_axis[1]);
     field_args(c, use_xi, comm_kind);
     c.E_tab = E_dev + row * B * 3;
     c.sigma = coulomb ? T : nullptr;
@@ -1270,11 +1352,12 @@ void Engine::rk4_step_tab(double dt, int ts, const bool use_axis[2], const bool 
 {
     state_dirty = true;  // the state it writes is checked by the next step or check_final_state
     StageUpdate u[4];
-    rk4_stages(dt, u);
-    evaluate_tab(y, ts, 0, use_axis, use_xi, u[0]);
-    evaluate_tab(aux, ts, 1, use_axis, use_xi, u[1]);
-    evaluate_tab(aux, ts, 1, use_axis, use_xi, u[2]);
-    evaluate_tab(aux, ts, 2, use_axis, use_xi, u[3]);
+    double2* in[4];
+    rk4_stages(dt, u, in);
+    evaluate_tab(in[0], ts, 0, use_axis, use_xi, u[0]);
+    evaluate_tab(in[1], ts, 1, use_axis, use_xi, u[1]);
+    evaluate_tab(in[2], ts, 1, use_axis, use_xi, u[2]);
+    evaluate_tab(in[3], ts, 2, use_axis, use_xi, u[3]);
 }
 
 // F^-1 diag(exp(i sign A.R)) F applied to (in + sum_d addc_d add_d), one
@@ -1374,11 +1457,12 @@ void Engine::rk4_step_peierls(double dt, const double* E3x3, const double* A3x3)
 {
     state_dirty = true;  // the state it writes is checked by the next step or check_final_state
     StageUpdate u[4];
-    rk4_stages(dt, u);
-    evaluate_peierls(y, E3x3 + 0, A3x3 + 0, u[0]);
-    evaluate_peierls(aux, E3x3 + 3, A3x3 + 3, u[1]);
-    evaluate_peierls(aux, E3x3 + 3, A3x3 + 3, u[2]);
-    evaluate_peierls(aux, E3x3 + 6, A3x3 + 6, u[3]);
+    double2* in[4];
+    rk4_stages(dt, u, in);
+    evaluate_peierls(in[0], E3x3 + 0, A3x3 + 0, u[0]);
+    evaluate_peierls(in[1], E3x3 + 3, A3x3 + 3, u[1]);
+    evaluate_peierls(in[2], E3x3 + 3, A3x3 + 3, u[2]);
+    evaluate_peierls(in[3], E3x3 + 6, A3x3 + 6, u[3]);
 }
 
 void Engine::ab_step_peierls(double dt, int order, const double* E3, const double* A3)

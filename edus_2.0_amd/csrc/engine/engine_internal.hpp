@@ -48,6 +48,8 @@ struct EngineOptions {
 
 class Batch;
 
+constexpr size_t kAxesSmallBytes = size_t(8) << 20;
+
 class Engine {
   public:
     explicit Engine(const edus_desc& d, const EngineOptions& opt = EngineOptions());
@@ -126,6 +128,22 @@ class Engine {
         if (grad_form_choice(N0, N1)) return grad_fused && plane_form(N0, N1);
         return !fft_choice[0].two_step || !fft_choice[1].two_step;
     }
+    // Both axes' derivatives in one launch, added by the commutator.  The same
+    // bytes as two passes (the second one reads the first one's result) without
+    // the second launch and its wait: 45 x 63, 21 planes 6 us instead of 10 (plane
+    // kernel), 120 x 120, 196 planes 34.6 instead of 41.9.  Line splits with a
+    // factor of 11 or above 12 need too many registers for the large grids (240 x
+    // 180, 100 planes: 63.7 us, two passes 69.5, but the step 4181 against 3740)
+    // and are taken up to a plane set of 8 MB.  Like plane_pass, not a function
+    // of the number of stacked instances.
+    bool axes_together() const
+    {
+        return !kgrad && !coulomb && !peierls && axes_available(N0, N1) && !(grad_form_choice(N0, N1) && grad_fused) &&
+               (!axes_wide(N0, N1) || size_t(npl) * Nk * sizeof(double2) <= kAxesSmallBytes);
+    }
+    // k-space gradient: the stencil's taps read by the commutator itself (RK4,
+    // whose stages never overwrite their input)
+    bool stencil_fused() const { return kst.size() <= 8; }
     // with exchange one launch instead of up to five (90 x 90, 64 planes: 19 us
     // instead of 32)
     bool plane_exchange() const { return plane_ok && (kgrad || !grad_form_choice(N0, N1) || grad_fused); }
@@ -178,8 +196,8 @@ class Engine {
     // record_order > 0: stage 1's right-hand side f(t_n, y_n) is also stored as
     // the newest Adams-Bashforth history entry of that order (RK4 start-up)
     void rk4_step(double dt, const double* E3x3, int record_order = 0);
-    // the stage updates of one RK4 step on y / acc / aux
-    void rk4_stages(double dt, StageUpdate u[4]) const;
+    // the stage updates of one RK4 step, and the input of each stage
+    void rk4_stages(double dt, StageUpdate u[4], double2* in[4]) const;
     // stacked instances: fields from the device tables at table step `ts`;
     // use_axis / use_xi switch off gradient axes and E.xi terms that are zero
     // for every instance of the chunk
@@ -219,7 +237,8 @@ class Engine {
     const double2* gradient(const double2* in, const double c[2], const double* ctab, bool use0, bool use1,
                             double2* fwd1 = nullptr, bool* fwd1_done = nullptr);
     // plane kernel: the derivative of in into D (deriv) and the exchange term into T (conv)
-    const double2* spectral_terms(const double2* in, const double c[2], const double* ctab, bool use0, bool use1);
+    void derivative_terms(CommArgs& c, const double cc[2], const double* ctab, const double* E, const double* E_tab,
+                          bool use0, bool use1);
     void plane_launch(const double2* in, bool deriv, const double c[2], const double* ctab, bool conv);
     void ensure_hist();
     // exchange term of in into T (+ Hartree diagonal); row_done: T already

@@ -61,17 +61,18 @@ struct AxisFFTArgs {
 // Per-stage update rule of the fused commutator kernel.  With f the
 // right-hand side at this k-point and element:
 //   out_f  = f                          (if out_f)
-//   out1   = x1 + b1 * f                (if out1)
+//   out1   = x1 + b1 * f                (if out1; see g1)
 //   out2   = x2 + b2 * f                (if out2)
 //   AB:    y  = y + sum_i c_i h_i  with h_0 = f, h_i = hist[i]  (if ab_order)
 struct StageUpdate {
     double2* out_f;
-    // RK: out1 = x1 + g1 (rho - x2) + b1 f and out2 = x2 + b2 f, rho the
-    // stage input (g1 lets a stage recover an earlier stage's b f term from
-    // rho - x2 instead of carrying it through another array)
+    // RK: out1 = x1 + b1 f and out2 = x2 + b2 f; with g1 out1 = rho +
+    // g1 (x1 - rho) + b1 f, or (g1_carried) x1 + g1 (rho - x2) + b1 f, rho the
+    // stage input: a stage recovers the earlier stages' f from their inputs
     const double2* x1; double2* out1; double b1;
     const double2* x2; double2* out2; double b2;
     double g1;
+    int g1_carried;
     int ab_order;
     const double2* hist[5];  // hist[0] unused (= f)
     double ab_c[5];
@@ -83,11 +84,25 @@ struct StageUpdate {
     double nf;
 };
 
+// k-space finite-difference gradient (gradient_space "k"): one stencil point
+// per mesh vector b of the shells in use: grid offset, shell weight, Cartesian b
+struct KStencilPoint {
+    int m0, m1;
+    double w;
+    double b[3];
+    int shell;
+};
+
 struct CommArgs {
     int Nk, P;
     int B;                    // instances stacked as [B][P][Nk] in every per-k array (0 or 1: one)
     const double2* rho;       // stage input, planes
     const double2* D;         // E.grad rho part (may be null)
+    const double2* D2;        // a second part, added to D (may be null)
+    // or E.grad rho by a finite-difference stencil over rho itself: nst > 0
+    // points kst (device), on the N0 x N1 mesh
+    const KStencilPoint* kst;
+    int nst, N0, N1;
     const double2* H0;
     const double2* xi[3];     // null where E_d == 0 or operator absent
     double E[3];
@@ -208,6 +223,14 @@ struct PlaneArgs {
     const double2* in_add[3];
     double in_add_c[3];
 };
+// Both axes' derivatives in one launch (plane_fft.hip): out[0] = F0^-1 i c0 R0 F0
+// in, out[1] = F1^-1 i c1 R1 F1 in, with in, out, P, N0, N1, the splits, tw0,
+// tw1 and the coefficients of a PlaneArgs from axes_args; for lengths with a
+// split into two factors of at most 16.
+bool axes_available(int N0, int N1);
+bool axes_wide(int N0, int N1);  // a factor of 11 or above 12 (more registers)
+PlaneArgs axes_args(int N0, int N1);
+void launch_axes(const PlaneArgs& a, hipStream_t s);
 bool plane_available(int N0, int N1);
 // grids on which the tuning chooses between the one-pass derivative
 // (plane_fft.hip, or grad_fused.hip where the plane does not fit) and axis passes
@@ -240,14 +263,7 @@ struct RotateArgs {
 };
 void launch_rotate(int nb, int in_layout, int kind, const RotateArgs& a, hipStream_t s);
 
-// k-space finite-difference gradient (gradient_space "k"): one stencil point
-// per mesh vector b of the shells in use: grid offset, shell weight, Cartesian b
-struct KStencilPoint {
-    int m0, m1;
-    double w;
-    double b[3];
-    int shell;
-};
+// k-space finite-difference gradient (gradient_space "k")
 std::vector<KStencilPoint> kgradient_stencil(const double A[3][3], int N0, int N1);
 // out = sum_b w_b (b.E) in(k + b) for every plane of B stacked instances;
 // E_tab ([B][3] on the device) replaces E when set

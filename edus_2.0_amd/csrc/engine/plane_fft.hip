@@ -91,7 +91,9 @@ struct PlaneAxis {
 // in memory with its own element and line strides.  Addresses advance by
 // wave-uniform strides (an index product per element would cost as much as
 // the transform: 32-bit integer multiplies run at a quarter of the FP64 rate).
-template <int NT, int MAXR, int S>
+// ROW: neighbouring lanes run along the line (coalesced where src or dst is a
+// row in memory) instead of across lines.
+template <int NT, int MAXR, int S, bool ROW = false>
 __device__ __forceinline__ void step_a(const PlaneAxis& ax, int tid, const double2* src, int se, int sl, double2* dst,
                                        int de, int dl)
 {
@@ -99,7 +101,14 @@ __device__ __forceinline__ void step_a(const PlaneAxis& ax, int tid, const doubl
         constexpr int R = decltype(r_)::value;
         const int RB = ax.RB, ntask = ax.lines * RB;
         for (int t = tid; t < ntask; t += NT) {
-            const int jb = fast_div(t, ax.inv_lines), line = t - jb * ax.lines;
+            int jb, line;
+            if (ROW) {
+                line = fast_div(t, ax.inv_RB);
+                jb = t - line * RB;
+            } else {
+                jb = fast_div(t, ax.inv_lines);
+                line = t - jb * ax.lines;
+            }
             const double2* p = src + (line * sl + jb * se);
             double2* q = dst + (line * dl + jb * de);
             double2 v[R];
@@ -300,6 +309,95 @@ __global__ void __launch_bounds__(NT, MAXR <= 12 ? 4 : 2) plane_kernel(PlaneArgs
     }
 }
 
+// Both axes' one-dimensional derivatives, their line groups side by side in one
+// launch: work-groups [0, nb0) take columns, the others rows, L lines each, and
+// the two results stay apart (the commutator adds them; either may be left
+// out).  On small grids, where
+// a launch costs what it computes, this saves the second launch and its wait
+// for the first.  Bound by latency there: three barriers and the launch.
+template <int NT, int MAXR>
+__global__ void __launch_bounds__(NT) axes_kernel(PlaneArgs a, int nb0, int L0, int L1)
+{
+    extern __shared__ double2 lds[];
+    const int N0 = a.N0, N1 = a.N1, Nk = N0 * N1, tid = threadIdx.x;
+    const bool col = int(blockIdx.x) < nb0;
+    const int n = col ? N0 : N1, RA = col ? a.RA0 : a.RA1, RB = col ? a.RB0 : a.RB1;
+    const int gs = col ? N1 : 1, gl = col ? 1 : N1;  // element and line strides in memory
+    long base;  // first element of the group's first line
+    int lines, plane0;
+    if (col) {
+        const int per = (N1 + L0 - 1) / L0;
+        plane0 = int(blockIdx.x) / per;
+        const int c = (int(blockIdx.x) - plane0 * per) * L0;
+        lines = min(L0, N1 - c);
+        base = long(plane0) * Nk + c;
+    } else {
+        const long row = long(blockIdx.x - nb0) * L1;
+        lines = int(min(long(L1), long(a.P) * N0 - row));
+        plane0 = int(row / N0);
+        base = row * N1;
+    }
+    const int row_in_plane = col ? 0 : int((base / N1) % N0);
+    const double2* src = a.in + base;
+    double2* dst = a.out[col ? 0 : 1] + base;
+    auto coef = [&](int line) {
+        if (!a.coef_tab) return col ? a.coef[0] : a.coef[1];
+        const int plane = col ? plane0 : plane0 + (row_in_plane + line) / N0;
+        return a.coef_tab[long(plane / a.ppi) * a.coef_stride + (col ? 0 : 1)];
+    };
+    if (RB == 1) {  // the whole line in one thread
+        with_radix<MAXR>(RA, [&](auto r_) {
+            constexpr int R = decltype(r_)::value;
+            for (int line = tid; line < lines; line += NT) {
+                const double2* p = src + line * gl;
+                double2* q = dst + line * gl;
+                const double c = coef(line);
+                double2 v[R];
+                sfor<R>([&](auto j_) {
+                    constexpr int j = decltype(j_)::value;
+                    v[j] = p[j * gs];
+                });
+                reg::rdft<R, -1>(v);
+                sfor<R>([&](auto j_) {
+                    constexpr int j = decltype(j_)::value;
+                    v[j] = cmul_i(v[j], c * double(gamma_centred(j, R)));
+                });
+                reg::rdft<R, 1>(v);
+                sfor<R>([&](auto j_) {
+                    constexpr int j = decltype(j_)::value;
+                    q[j * gs] = v[j];
+                });
+            }
+        });
+        return;
+    }
+    double2* tw = lds;
+    double2* buf = lds + n;
+    const double2* twg = col ? a.tw0 : a.tw1;
+    for (int i = tid; i < n; i += NT) tw[i] = twg[i];
+    const int es = col ? L0 : 1, ls = col ? 1 : (n | 1);  // strides in LDS
+    const PlaneAxis ax{n, RA, RB, lines, es, ls, 1.0f / float(lines), 1.0f / float(RB), tw};
+    __syncthreads();
+    if (col)
+        step_a<NT, MAXR, -1>(ax, tid, src, gs, gl, buf, es, ls);
+    else
+        step_a<NT, MAXR, -1, true>(ax, tid, src, gs, gl, buf, es, ls);
+    __syncthreads();
+    step_b<NT, MAXR, 0>(ax, tid, buf, [&](int line, int ka, auto& u) {
+        constexpr int R = sizeof(u) / sizeof(double2);
+        const double c = coef(line);
+        sfor<R>([&](auto k_) {
+            constexpr int k = decltype(k_)::value;
+            u[k] = cmul_i(u[k], c * double(gamma_centred(ka + RA * k, n)));
+        });
+    });
+    __syncthreads();
+    if (col)
+        step_a<NT, MAXR, 1>(ax, tid, buf, es, ls, dst, gs, gl);
+    else
+        step_a<NT, MAXR, 1, true>(ax, tid, buf, es, ls, dst, gs, gl);
+}
+
 // W[f0 * N1 + f1] of every plane into the order the convolution reads it:
 // Wp[p1 * N0 + p0], the frequencies at positions p0, p1 of the two axes
 __global__ void plane_permute_kernel(const double* __restrict__ W, double* __restrict__ Wp, long total, int N0, int N1,
@@ -345,6 +443,13 @@ void launch_plane_nt(const PlaneArgs& a, int blocks, size_t lds, hipStream_t s)
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), lds, s, a);
 }
 
+bool wide_radix(const PlaneArgs& a)
+{
+    for (int r : {a.RA0, a.RB0, a.RA1, a.RB1})
+        if (r > 12 || r == 11) return true;
+    return false;
+}
+
 size_t plane_lds(int N0, int N1, bool phase)
 {
     return size_t(N0 * (N1 | 1) + (phase ? 2 : 1) * (N0 + N1)) * sizeof(double2);
@@ -386,8 +491,7 @@ void launch_plane_shape(const PlaneArgs& a, hipStream_t s)
     // as many threads as give a step about one round of tasks (us for 256, 512,
     // 1024 threads: 30 x 30, 4 planes 6.2, 6.2, 6.5; 60 x 66, 25 planes 13.7,
     // 11.9, 12.2; 90 x 90 with exchange, 64 planes 25.0, 22.1, 18.9)
-    bool wide = false;
-    for (int r : {a.RA0, a.RB0, a.RA1, a.RB1}) wide = wide || r > 12 || r == 11;
+    const bool wide = wide_radix(a);
     const int Nk = a.N0 * a.N1;
     if (wide)
         launch_plane_nt<512, 16, PHASE>(a, blocks, lds, s);
@@ -405,6 +509,47 @@ void launch_plane(const PlaneArgs& a, hipStream_t s)
         launch_plane_shape<true>(a, s);
     else
         launch_plane_shape<false>(a, s);
+}
+
+bool axes_available(int N0, int N1)
+{
+    int b, c;
+    return split_line(N0, b, c) && split_line(N1, b, c);
+}
+
+bool axes_wide(int N0, int N1) { return wide_radix(axes_args(N0, N1)); }
+
+PlaneArgs axes_args(int N0, int N1)
+{
+    PlaneArgs a{};
+    a.N0 = N0;
+    a.N1 = N1;
+    split_line(N0, a.RA0, a.RB0);
+    split_line(N1, a.RA1, a.RB1);
+    return a;
+}
+
+void launch_axes(const PlaneArgs& a, hipStream_t s)
+{
+    constexpr int NT = 256;
+    // about one task per thread and step, columns in whole 128-byte runs, within
+    // the 64 KB of LDS that need no raised limit
+    auto lines = [](int n, int RA, int RB) {
+        if (RB == 1) return NT;
+        const int most = (64 * 1024 / int(sizeof(double2)) - n) / (n | 1);
+        return std::max(1, std::min(NT / std::max(RA, RB), most));
+    };
+    int L0 = std::min(lines(a.N0, a.RA0, a.RB0), a.N1);
+    if (L0 > 8 && L0 < a.N1) L0 = L0 / 8 * 8;
+    const int L1 = lines(a.N1, a.RA1, a.RB1);
+    const int nb0 = a.out[0] ? a.P * ((a.N1 + L0 - 1) / L0) : 0;
+    const int nb1 = a.out[1] ? int((long(a.P) * a.N0 + L1 - 1) / L1) : 0;
+    const size_t lds = sizeof(double2) * std::max(a.RB0 > 1 ? a.N0 + a.N0 * L0 : 0,
+                                                  a.RB1 > 1 ? a.N1 + (a.N1 | 1) * L1 : 0);
+    if (wide_radix(a))
+        hipLaunchKernelGGL((axes_kernel<NT, 16>), dim3(nb0 + nb1), dim3(NT), lds, s, a, nb0, L0, L1);
+    else
+        hipLaunchKernelGGL((axes_kernel<NT, 12>), dim3(nb0 + nb1), dim3(NT), lds, s, a, nb0, L0, L1);
 }
 
 void launch_plane_permute(const double* W, double* Wp, int P, int N0, int N1, hipStream_t s)

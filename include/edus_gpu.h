@@ -197,7 +197,8 @@ int edus_graph(edus_ctx* ctx, int steps_per_graph);
 /* Kernel timing with HIP events on the context stream.  When enabled, every
  * launch of the named kernel class is bracketed by events; edus_timing_get
  * returns the summed milliseconds and launch count since the last reset.
- * Classes: "grad_col", "grad_row", "grad_fused", "kgrad", "comm", "hf_row",
+ * Classes: "grad_col", "grad_row", "grad_axes" (both axes' derivatives in one
+ * launch, two results that "comm" adds), "grad_fused", "kgrad", "comm", "hf_row",
  * "hf_col", "hf_plane" (the exchange term, with the derivative where the field
  * has one, one work-group per plane), "peierls_col", "peierls_row",
  * "peierls_plane", "rotate". */
@@ -222,10 +223,10 @@ int edus_timing_get(edus_ctx* ctx, const char* kernel_class, double* total_ms, l
  *   grad_fused     1: the spectral derivative in one pass per plane (one
  *                  work-group holds a plane: grids 120 x 120, 96 x 96,
  *                  90 x 90, 48 x 48; on the last three the exchange term too);
- *                  0: axis passes through work plane sets.  Other grids have
- *                  no choice (0): with exchange, or where an axis has no
- *                  two-step kernel, planes that fit in LDS go one work-group
- *                  per plane, the rest take axis passes.
+ *                  0: axis passes, both axes' in one launch.  Other grids
+ *                  have no choice (0): with exchange planes that fit in LDS go
+ *                  one work-group per plane; without, both axes' passes share a
+ *                  launch where the line lengths' factors allow it.
  *   tri_fields     1: the MFMA commutator engines read H0(k) and r_d(k) from
  *                  copies of their upper triangles, the lower elements as
  *                  conjugates (0.54 of the bytes at nb = 14); 0: from every

@@ -1,9 +1,9 @@
-"""GPU: the spectral passes with a whole plane in LDS (one work-group per
-plane), against the oracle, on the grids that take them: an axis without a
-two-step kernel, every exchange grid whose planes fit, and the Peierls phase.
-The lengths cover one-step lines (at most 16), both orders of a short and a
-long axis, every radix of the kernel, the largest plane that fits in LDS and
-the first one that does not.
+"""GPU: the spectral passes of plane_fft.hip against the oracle: both axes'
+derivatives in one launch (most grids), and one work-group per plane in LDS
+(exchange, the Peierls phase, and derivatives of large fields on grids whose
+line splits have large factors).  The lengths cover one-step lines (at most
+16), both orders of a short and a long axis, every radix of the kernels, and
+for exchange and phase planes up to the limit of LDS.
 
 Bar: one right-hand side within 1e-11 relative (as the other parity tests)."""
 import os
@@ -58,6 +58,18 @@ def test_derivative(model_dir, grid):
     o = oracle_py.Oracle(p)
     eng = _engine(o, p)
     rho = _rho(o, 4)
+    for E in _fields(o):
+        ref = o.rhs_E(E, rho)
+        assert np.abs(eng.rhs(E, rho) - ref).max() <= 1e-11 * max(1.0, np.abs(ref).max())
+
+
+def test_derivative_in_lds(model_dir):
+    """14 bands on 66 x 45: above the field size up to which factors of 11 take
+    the one-launch form of both axes."""
+    p = _model("ipa14_hex120", model_dir, (66, 45))
+    o = oracle_py.Oracle(p)
+    eng = _engine(o, p)
+    rho = _rho(o, 9)
     for E in _fields(o):
         ref = o.rhs_E(E, rho)
         assert np.abs(eng.rhs(E, rho) - ref).max() <= 1e-11 * max(1.0, np.abs(ref).max())
