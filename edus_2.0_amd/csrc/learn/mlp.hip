@@ -26,6 +26,8 @@ typedef float flt4 __attribute__((ext_vector_type(4)));
 
 constexpr int kTile = 64;   // rows and columns of C per work-group
 constexpr int kKStep = 16;  // K per MFMA
+constexpr int kStage = 64;  // K per pass through LDS
+constexpr int kLd = kStage + 4;  // LDS row of an operand: 34 words, the fragment reads of 16 rows spread over the banks
 
 struct GemmArgs {
     const uint16_t* A;
@@ -45,10 +47,85 @@ struct GemmArgs {
     int ldm;
 };
 
+// 4 consecutive BF16 values from p (8-byte aligned when VEC), those at index
+// first + e < n
+template <bool VEC>
+__device__ inline ushort4 load4(const uint16_t* p, long first, long n)
+{
+    if (VEC && first + 4 <= n) return *reinterpret_cast<const ushort4*>(p);
+    ushort4 v = make_ushort4(0, 0, 0, 0);
+    if (first < n) v.x = p[0];
+    if (first + 1 < n) v.y = p[1];
+    if (first + 2 < n) v.z = p[2];
+    if (first + 3 < n) v.w = p[3];
+    return v;
+}
+
+// One operand's 64 x kStage tile in registers, then in LDS as s[row][k].
+// KROW: k is the contiguous index in memory (a thread takes 16 k of one row);
+// otherwise the rows are (a thread takes 8 rows at two adjacent k and writes
+// pairs).  ones: a row that reads 1.0.
+template <bool KROW, bool VEC>
+struct Tile {
+    ushort4 v[4];
+    __device__ void load(const uint16_t* X, long sr, long sk, int r0, int rows, int k0, int ke, int ones)
+    {
+        const int t = threadIdx.x;
+        if (KROW) {
+            const int r = r0 + (t >> 2), k = k0 + (t & 3) * 16;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = make_ushort4(0, 0, 0, 0);
+                if (r < rows) v[e] = load4<VEC>(X + long(r) * sr + k + 4 * e, k + 4 * e, ke);
+            }
+        } else {
+            const int r = r0 + (t & 7) * 8, k = k0 + (t >> 3) * 2;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int kk = k + (e >> 1), rr = r + (e & 1) * 4;
+                v[e] = make_ushort4(0, 0, 0, 0);
+                if (kk < ke) {
+                    // the row of ones lies behind the operand's own rows
+                    v[e] = load4<VEC>(X + long(kk) * sk + rr, rr, ones >= 0 ? ones : rows);
+                    const int o = ones - rr;
+                    if (ones >= 0 && o >= 0 && o < 4) reinterpret_cast<uint16_t*>(&v[e])[o] = 0x3f80;
+                }
+            }
+        }
+    }
+    __device__ void store(uint16_t (*s)[kLd]) const
+    {
+        const int t = threadIdx.x;
+        if (KROW) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                *reinterpret_cast<ushort4*>(&s[t >> 2][(t & 3) * 16 + 4 * e]) = v[e];
+        } else {
+            const int r = (t & 7) * 8, k = (t >> 3) * 2;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const ushort4 a = v[h], b = v[2 + h];
+                const uint16_t x[4] = {a.x, a.y, a.z, a.w}, y[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    *reinterpret_cast<uint32_t*>(&s[r + 4 * h + e][k]) = uint32_t(x[e]) | (uint32_t(y[e]) << 16);
+            }
+        }
+    }
+};
+
+// C = A B on 64 x 64 tiles, 16 rows of a tile per wave.  Both operands pass
+// through LDS with k contiguous (whatever their order in memory), 64 k per
+// barrier pair, the next 64 loaded into registers meanwhile; a fragment is one
+// 8-byte read.  The products are summed over k in steps of 16 in ascending
+// order, whatever the staging.  Bound by the latency of its few stages and, on
+// small shapes, by the launch: 8192 rows, 256 x 256, 14 us; with one 2-byte element
+// per load and read and 16 k per barrier it took 32 to 60.
+template <bool AK, bool VEC>
 __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g)
 {
-    __shared__ uint16_t sA[kTile][kKStep + 4];
-    __shared__ uint16_t sB[kKStep][kTile + 4];
+    __shared__ __align__(16) uint16_t sA[kTile][kLd];
+    __shared__ __align__(16) uint16_t sB[kTile][kLd];
     const int m0 = blockIdx.x * kTile, n0 = blockIdx.y * kTile;
     const int kb = blockIdx.z * g.kchunk;
     const int ke = min(g.K, kb + g.kchunk);
@@ -58,33 +135,27 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmArgs g)
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[t] = flt4{0.f, 0.f, 0.f, 0.f};
 
-    for (int k0 = kb; k0 < ke; k0 += kKStep) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int idx = threadIdx.x + e * 256;  // 64 x 16 tile of A
-            const int r = idx >> 4, c = idx & 15;
-            const int m = m0 + r, k = k0 + c;
-            uint16_t v = 0;
-            if (m < g.M && k < ke) v = (m == g.ones_row) ? uint16_t(0x3f80) : g.A[m * g.sam + k * g.sak];
-            sA[r][c] = v;
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int idx = threadIdx.x + e * 256;  // 16 x 64 tile of B
-            const int r = idx >> 6, c = idx & 63;
-            const int k = k0 + r, n = n0 + c;
-            sB[r][c] = (k < ke && n < g.N) ? g.B[k * g.sbk + n * g.sbn] : uint16_t(0);
-        }
+    Tile<AK, VEC> ta;
+    Tile<false, VEC> tb;
+    ta.load(g.A, g.sam, g.sak, m0, g.M, kb, ke, g.ones_row);
+    tb.load(g.B, g.sbn, g.sbk, n0, g.N, kb, ke, -1);
+    for (int k0 = kb; k0 < ke; k0 += kStage) {
+        ta.store(sA);
+        tb.store(sB);
         __syncthreads();
-        bf16x4 a;
+        if (k0 + kStage < ke) {
+            ta.load(g.A, g.sam, g.sak, m0, g.M, k0 + kStage, ke, g.ones_row);
+            tb.load(g.B, g.sbn, g.sbk, n0, g.N, k0 + kStage, ke, -1);
+        }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) a[e] = short(sA[16 * wave + i][4 * q + e]);
+        for (int ks = 0; ks < kStage; ks += kKStep) {
+            if (k0 + ks >= ke) break;
+            const bf16x4 a = *reinterpret_cast<const bf16x4*>(&sA[16 * wave + i][ks + 4 * q]);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            bf16x4 b;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) b[e] = short(sB[4 * q + e][16 * t + i]);
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[t], 0, 0, 0);
+            for (int t = 0; t < 4; ++t) {
+                const bf16x4 b = *reinterpret_cast<const bf16x4*>(&sB[16 * t + i][ks + 4 * q]);
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[t], 0, 0, 0);
+            }
         }
         __syncthreads();
     }
@@ -182,7 +253,39 @@ __global__ void to_bf16_kernel(const float* __restrict__ W, int rows, int cols, 
     WbT[size_t(c) * rows + r] = b;
 }
 
+// x rounded to BF16, four values per thread
+__global__ void __launch_bounds__(256) round_bf16_kernel(const float* __restrict__ x, long n, uint16_t* __restrict__ b)
+{
+    const long i = (blockIdx.x * 256L + threadIdx.x) * 4;
+    if (i + 4 <= n) {
+        const float4 v = *reinterpret_cast<const float4*>(x + i);
+        *reinterpret_cast<ushort4*>(b + i) = make_ushort4(f2bf(v.x), f2bf(v.y), f2bf(v.z), f2bf(v.w));
+    } else {
+        for (long e = i; e < n; ++e) b[e] = f2bf(x[e]);
+    }
+}
+
 int cdiv(long a, long b) { return int((a + b - 1) / b); }
+
+void launch_gemm(const GemmArgs& g, int nz, hipStream_t s)
+{
+    const dim3 grid(cdiv(g.M, kTile), cdiv(g.N, kTile), nz);
+    const bool ak = g.sak == 1;
+    if (g.sbn != 1 || (!ak && g.sam != 1) || (ak && g.ones_row >= 0))
+        throw EngineError(EDUS_ERR_ARG, "GEMM operand order not supported");
+    // 8-byte loads where every row starts on 8 bytes; kchunk is a multiple of 16
+    const long ld = ak ? g.sam : g.sak;
+    const bool vec = ld % 4 == 0 && g.sbk % 4 == 0 && reinterpret_cast<uintptr_t>(g.A) % 8 == 0 &&
+                     reinterpret_cast<uintptr_t>(g.B) % 8 == 0;
+    if (ak && vec)
+        hipLaunchKernelGGL((gemm_bf16_kernel<true, true>), grid, dim3(256), 0, s, g);
+    else if (ak)
+        hipLaunchKernelGGL((gemm_bf16_kernel<true, false>), grid, dim3(256), 0, s, g);
+    else if (vec)
+        hipLaunchKernelGGL((gemm_bf16_kernel<false, true>), grid, dim3(256), 0, s, g);
+    else
+        hipLaunchKernelGGL((gemm_bf16_kernel<false, false>), grid, dim3(256), 0, s, g);
+}
 
 }  // namespace
 
@@ -210,7 +313,7 @@ void launch_gemm_bf16(const uint16_t* A, long sam, long sak, const uint16_t* B, 
     g.ldcb = ldcb;
     g.mul = mul;
     g.ldm = N;
-    hipLaunchKernelGGL(gemm_bf16_kernel, dim3(cdiv(M, kTile), cdiv(N, kTile), 1), dim3(256), 0, s, g);
+    launch_gemm(g, 1, s);
 }
 
 void* Mlp::alloc(size_t bytes)
@@ -258,6 +361,37 @@ Mlp::~Mlp()
 {
     (void)hipStreamSynchronize(s);
     for (void* p : owned) (void)hipFree(p);
+    for (auto& b : io) (void)hipFree(b.p);
+}
+
+// Input buffer k of the calls on host arrays, at least `bytes` long: kept from
+// call to call, replaced when a call needs more, released with the network.
+void* Mlp::io_buffer(int k, size_t bytes)
+{
+    IoBuffer& b = io[k];
+    if (bytes > b.bytes) {
+        HIP_CHECK(hipStreamSynchronize(s));  // nothing queued reads the old one
+        HIP_CHECK(hipFree(b.p));
+        b.p = nullptr;
+        b.bytes = 0;
+        HIP_CHECK(hipMalloc(&b.p, bytes));
+        b.bytes = bytes;
+    }
+    return b.p;
+}
+
+// n host values rounded to BF16 on the device, through a staging buffer of at
+// most 16 MB (rounding 8192 x 148 values on one host core took 268 us, the
+// copy of the FP32 values instead of the rounded ones takes 60 us more)
+void Mlp::upload_bf16(const float* host, size_t n, uint16_t* dst)
+{
+    const size_t chunk = std::min<size_t>(n, size_t(4) << 20);
+    float* st = static_cast<float*>(io_buffer(kIoStage, chunk * sizeof(float)));
+    for (size_t o = 0; o < n; o += chunk) {
+        const size_t m = std::min(chunk, n - o);
+        HIP_CHECK(hipMemcpyAsync(st, host + o, m * sizeof(float), hipMemcpyHostToDevice, s));
+        hipLaunchKernelGGL(round_bf16_kernel, dim3(cdiv(long(m), 1024)), dim3(256), 0, s, st, long(m), dst + o);
+    }
 }
 
 void Mlp::set_params(const float* host)
@@ -324,7 +458,9 @@ void Mlp::forward(const uint16_t* X, int M, float* Y, bool keep)
 void Mlp::weight_grad(const uint16_t* A, int lda, const uint16_t* D, int ldd, int M, int K, int N, float* dW,
                       float* db)
 {
-    const int nz = std::max(1, std::min(64, M / 1024));
+    // split-K: 256 rows per part, so that a few thousand rows fill the chip (8192
+    // rows, 256 x 256 weights: 47 us in 8 parts of 1024 rows)
+    const int nz = std::max(1, std::min(64, M / 256));
     const int kchunk = ((cdiv(M, nz) + kKStep - 1) / kKStep) * kKStep;
     const int nzz = cdiv(M, kchunk);
     ensure_partial(size_t(nzz) * (K + 1) * N);
@@ -342,7 +478,7 @@ void Mlp::weight_grad(const uint16_t* A, int lda, const uint16_t* D, int ldd, in
     g.ones_row = K;
     g.C = partial;
     g.ldc = N;
-    hipLaunchKernelGGL(gemm_bf16_kernel, dim3(cdiv(K + 1, kTile), cdiv(N, kTile), nzz), dim3(256), 0, s, g);
+    launch_gemm(g, nzz, s);
     hipLaunchKernelGGL(reduce_partials_kernel, dim3(cdiv(long(K + 1) * N, 256)), dim3(256), 0, s, partial, nzz, K, N,
                        dW, db);
 }

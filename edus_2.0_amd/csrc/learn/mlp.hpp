@@ -64,7 +64,19 @@ class Mlp {
     void get_params(float* host) const;
     void get_grads(float* host) const;
 
+    // device buffers of the calls on host arrays: inputs, targets, loss values
+    // and the FP32 staging of upload_bf16
+    enum { kIoX = 0, kIoT = 1, kIoLoss = 2, kIoStage = 3, kIoCount = 4 };
+    void* io_buffer(int k, size_t bytes);
+    void upload_bf16(const float* host, size_t n, uint16_t* dst);
+    const float* output() const { return Ybuf; }  // of the last forward with Y null
+
   private:
+    struct IoBuffer {
+        void* p = nullptr;
+        size_t bytes = 0;
+    };
+    IoBuffer io[kIoCount];
     std::vector<void*> owned;
     int cap_rows = 0;
     uint16_t *H1 = nullptr, *H2 = nullptr, *dYb = nullptr, *dZ2 = nullptr, *dZ1 = nullptr;

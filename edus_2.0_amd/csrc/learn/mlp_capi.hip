@@ -34,17 +34,6 @@ __global__ void gather_rows_kernel(const uint16_t* __restrict__ X, const float* 
 
 using edus::guarded;
 
-namespace {
-
-std::vector<uint16_t> to_bf16(const float* x, size_t n)
-{
-    std::vector<uint16_t> b(n);
-    for (size_t i = 0; i < n; ++i) b[i] = edus::f2bf(x[i]);
-    return b;
-}
-
-}  // namespace
-
 extern "C" {
 
 edus_mlp* edus_mlp_create(int din, int dh, int dout, unsigned long long seed)
@@ -95,13 +84,13 @@ int edus_mlp_forward(edus_mlp* m, int rows, const float* X, float* Y)
     EDUS_REQUIRE(m && X && Y && rows >= 0);
     return guarded([&] {
         edus::Mlp& net = *m->h.m;
-        const auto xb = to_bf16(X, size_t(rows) * net.din);
-        edus::MlpHandle tmp;  // scratch for this call
-        uint16_t* dX = tmp.dev<uint16_t>(xb.size());
-        float* dY = tmp.dev<float>(size_t(rows) * net.dout);
-        HIP_CHECK(hipMemcpyAsync(dX, xb.data(), xb.size() * sizeof(uint16_t), hipMemcpyHostToDevice, net.s));
-        net.forward(dX, rows, dY, false);
-        HIP_CHECK(hipMemcpyAsync(Y, dY, size_t(rows) * net.dout * sizeof(float), hipMemcpyDeviceToHost, net.s));
+        if (rows == 0) return;
+        const size_t nx = size_t(rows) * net.din;
+        auto* dX = static_cast<uint16_t*>(net.io_buffer(edus::Mlp::kIoX, nx * sizeof(uint16_t)));
+        net.upload_bf16(X, nx, dX);
+        net.forward(dX, rows, nullptr, false);
+        HIP_CHECK(hipMemcpyAsync(Y, net.output(), size_t(rows) * net.dout * sizeof(float), hipMemcpyDeviceToHost,
+                                 net.s));
         HIP_CHECK(hipStreamSynchronize(net.s));
     });
 }
@@ -111,14 +100,13 @@ int edus_mlp_gradients(edus_mlp* m, int rows, const float* X, const float* T, fl
     EDUS_REQUIRE(m && X && T && grads && rows > 0);
     return guarded([&] {
         edus::Mlp& net = *m->h.m;
-        const auto xb = to_bf16(X, size_t(rows) * net.din);
-        edus::MlpHandle tmp;
-        uint16_t* dX = tmp.dev<uint16_t>(xb.size());
-        float* dT = tmp.dev<float>(size_t(rows) * net.dout);
-        float* dL = tmp.dev<float>(1);
-        HIP_CHECK(hipMemcpyAsync(dX, xb.data(), xb.size() * sizeof(uint16_t), hipMemcpyHostToDevice, net.s));
-        HIP_CHECK(hipMemcpyAsync(dT, T, size_t(rows) * net.dout * sizeof(float), hipMemcpyHostToDevice, net.s));
+        const size_t nx = size_t(rows) * net.din, nt = size_t(rows) * net.dout;
+        auto* dX = static_cast<uint16_t*>(net.io_buffer(edus::Mlp::kIoX, nx * sizeof(uint16_t)));
+        auto* dT = static_cast<float*>(net.io_buffer(edus::Mlp::kIoT, nt * sizeof(float)));
+        auto* dL = static_cast<float*>(net.io_buffer(edus::Mlp::kIoLoss, sizeof(float)));
+        net.upload_bf16(X, nx, dX);
         net.forward(dX, rows, nullptr, true);
+        HIP_CHECK(hipMemcpyAsync(dT, T, nt * sizeof(float), hipMemcpyHostToDevice, net.s));
         net.backward(dX, dT, rows, dL);
         float l = 0.f;
         HIP_CHECK(hipMemcpyAsync(&l, dL, sizeof(float), hipMemcpyDeviceToHost, net.s));
@@ -138,16 +126,16 @@ int edus_mlp_train(edus_mlp* m, int rows, const float* X, const float* T, int ep
     return guarded([&] {
         edus::Mlp& net = *m->h.m;
         batch = std::min(batch, rows);
-        const auto xb = to_bf16(X, size_t(rows) * net.din);
+        const size_t nx = size_t(rows) * net.din;
         edus::MlpHandle tmp;
-        uint16_t* dX = tmp.dev<uint16_t>(xb.size());
+        uint16_t* dX = tmp.dev<uint16_t>(nx);
         float* dT = tmp.dev<float>(size_t(rows) * net.dout);
         uint16_t* bX = tmp.dev<uint16_t>(size_t(batch) * net.din);
         float* bT = tmp.dev<float>(size_t(batch) * net.dout);
         const int nb = rows / batch;  // full batches per epoch
         float* dL = tmp.dev<float>(size_t(std::max(nb, 1)));
         int* didx = tmp.dev<int>(size_t(rows));
-        HIP_CHECK(hipMemcpyAsync(dX, xb.data(), xb.size() * sizeof(uint16_t), hipMemcpyHostToDevice, net.s));
+        net.upload_bf16(X, nx, dX);
         HIP_CHECK(hipMemcpyAsync(dT, T, size_t(rows) * net.dout * sizeof(float), hipMemcpyHostToDevice, net.s));
         std::vector<int> perm(rows);
         std::iota(perm.begin(), perm.end(), 0);
