@@ -130,11 +130,12 @@ class Engine {
     }
     // Both axes' derivatives in one launch, added by the commutator.  The same
     // bytes as two passes (the second one reads the first one's result) without
-    // the second launch and its wait: 45 x 63, 21 planes 6 us instead of 10 (plane
-    // kernel), 120 x 120, 196 planes 34.6 instead of 41.9.  Line splits with a
-    // factor of 11 or above 12 need too many registers for the large grids (240 x
-    // 180, 100 planes: 63.7 us, two passes 69.5, but the step 4181 against 3740)
-    // and are taken up to a plane set of 8 MB.  Like plane_pass, not a function
+    // the second launch and its wait: 45 x 63, 21 planes 4.8 us instead of 10 (plane
+    // kernel), 120 x 120, 196 planes 31.8 instead of 41.9.  Line splits with a
+    // factor of 11 or above 12 are taken up to a plane set of 8 MB: on large grids
+    // the second result, one more array in the cache behind HBM, costs the
+    // commutator more than the launch gains (240 x 180, 100 planes: 48.3 us, two
+    // passes 69.5, but ten steps 4099 against 3781).  Like plane_pass, not a function
     // of the number of stacked instances.
     bool axes_together() const
     {

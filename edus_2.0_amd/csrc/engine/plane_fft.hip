@@ -48,6 +48,7 @@ namespace {
 using reg::sfor;
 
 constexpr size_t kPlaneLds = 160 * 1024;
+constexpr int kAxesMaxThreads = 256;
 
 // q = t / d for 0 <= t < 2^20 and 0 < d < 2^12, inv = 1 / d in FP32: t + 1/2
 // is at least 1/2 away from any multiple of d, far above the rounding
@@ -92,15 +93,17 @@ struct PlaneAxis {
 // wave-uniform strides (an index product per element would cost as much as
 // the transform: 32-bit integer multiplies run at a quarter of the FP64 rate).
 // ROW: neighbouring lanes run along the line (coalesced where src or dst is a
-// row in memory) instead of across lines.
+// row in memory) instead of across lines.  NT threads, or with NT = 0 as many as
+// the work-group has.
 template <int NT, int MAXR, int S, bool ROW = false>
 __device__ __forceinline__ void step_a(const PlaneAxis& ax, int tid, const double2* src, int se, int sl, double2* dst,
                                        int de, int dl)
 {
+    const int nt = NT ? NT : blockDim.x;
     with_radix<MAXR>(ax.RA, [&](auto r_) {
         constexpr int R = decltype(r_)::value;
         const int RB = ax.RB, ntask = ax.lines * RB;
-        for (int t = tid; t < ntask; t += NT) {
+        for (int t = tid; t < ntask; t += nt) {
             int jb, line;
             if (ROW) {
                 line = fast_div(t, ax.inv_RB);
@@ -145,10 +148,11 @@ __device__ __forceinline__ void step_a(const PlaneAxis& ax, int tid, const doubl
 template <int NT, int MAXR, int S, class Mul>
 __device__ __forceinline__ void step_b(const PlaneAxis& ax, int tid, double2* pl, Mul mul)
 {
+    const int nt = NT ? NT : blockDim.x;
     with_radix<MAXR>(ax.RB, [&](auto r_) {
         constexpr int R = decltype(r_)::value;
         const int ntask = ax.lines * ax.RA;
-        for (int t = tid; t < ntask; t += NT) {
+        for (int t = tid; t < ntask; t += nt) {
             const int ka = fast_div(t, ax.inv_lines), line = t - ka * ax.lines;
             const int es = ax.estr;
             double2* p = pl + (line * ax.lstr + ka * R * es);
@@ -314,9 +318,11 @@ __global__ void __launch_bounds__(NT, MAXR <= 12 ? 4 : 2) plane_kernel(PlaneArgs
 // the two results stay apart (the commutator adds them; either may be left
 // out).  On small grids, where
 // a launch costs what it computes, this saves the second launch and its wait
-// for the first.  Bound by latency there: three barriers and the launch.
-template <int NT, int MAXR>
-__global__ void __launch_bounds__(NT) axes_kernel(PlaneArgs a, int nb0, int L0, int L1)
+// for the first.  Bound by latency there: three barriers and the launch.  On
+// large ones by memory and the lanes at work (axes_best_shape): 120 x 120, 196
+// planes 31.8 us, 5.7 TB/s of its two reads and two writes.
+template <int MAXR>
+__global__ void __launch_bounds__(kAxesMaxThreads, MAXR <= 12 ? 4 : 3) axes_kernel(PlaneArgs a, int nb0, int L0, int L1)
 {
     extern __shared__ double2 lds[];
     const int N0 = a.N0, N1 = a.N1, Nk = N0 * N1, tid = threadIdx.x;
@@ -348,7 +354,7 @@ __global__ void __launch_bounds__(NT) axes_kernel(PlaneArgs a, int nb0, int L0, 
     if (RB == 1) {  // the whole line in one thread
         with_radix<MAXR>(RA, [&](auto r_) {
             constexpr int R = decltype(r_)::value;
-            for (int line = tid; line < lines; line += NT) {
+            for (int line = tid; line < lines; line += blockDim.x) {
                 const double2* p = src + line * gl;
                 double2* q = dst + line * gl;
                 const double c = coef(line);
@@ -374,16 +380,16 @@ __global__ void __launch_bounds__(NT) axes_kernel(PlaneArgs a, int nb0, int L0, 
     double2* tw = lds;
     double2* buf = lds + n;
     const double2* twg = col ? a.tw0 : a.tw1;
-    for (int i = tid; i < n; i += NT) tw[i] = twg[i];
+    for (int i = tid; i < n; i += blockDim.x) tw[i] = twg[i];
     const int es = col ? L0 : 1, ls = col ? 1 : (n | 1);  // strides in LDS
     const PlaneAxis ax{n, RA, RB, lines, es, ls, 1.0f / float(lines), 1.0f / float(RB), tw};
     __syncthreads();
     if (col)
-        step_a<NT, MAXR, -1>(ax, tid, src, gs, gl, buf, es, ls);
+        step_a<0, MAXR, -1>(ax, tid, src, gs, gl, buf, es, ls);
     else
-        step_a<NT, MAXR, -1, true>(ax, tid, src, gs, gl, buf, es, ls);
+        step_a<0, MAXR, -1, true>(ax, tid, src, gs, gl, buf, es, ls);
     __syncthreads();
-    step_b<NT, MAXR, 0>(ax, tid, buf, [&](int line, int ka, auto& u) {
+    step_b<0, MAXR, 0>(ax, tid, buf, [&](int line, int ka, auto& u) {
         constexpr int R = sizeof(u) / sizeof(double2);
         const double c = coef(line);
         sfor<R>([&](auto k_) {
@@ -393,9 +399,9 @@ __global__ void __launch_bounds__(NT) axes_kernel(PlaneArgs a, int nb0, int L0, 
     });
     __syncthreads();
     if (col)
-        step_a<NT, MAXR, 1>(ax, tid, buf, es, ls, dst, gs, gl);
+        step_a<0, MAXR, 1>(ax, tid, buf, es, ls, dst, gs, gl);
     else
-        step_a<NT, MAXR, 1, true>(ax, tid, buf, es, ls, dst, gs, gl);
+        step_a<0, MAXR, 1, true>(ax, tid, buf, es, ls, dst, gs, gl);
 }
 
 // W[f0 * N1 + f1] of every plane into the order the convolution reads it:
@@ -529,27 +535,71 @@ PlaneArgs axes_args(int N0, int N1)
     return a;
 }
 
-void launch_axes(const PlaneArgs& a, hipStream_t s)
+namespace {
+
+// Threads and lines of an axes_kernel launch
+struct AxesShape {
+    int nt, L0, L1;
+    size_t lds;
+};
+
+AxesShape axes_shape(const PlaneArgs& a, int nt)
 {
-    constexpr int NT = 256;
     // about one task per thread and step, columns in whole 128-byte runs, within
     // the 64 KB of LDS that need no raised limit
-    auto lines = [](int n, int RA, int RB) {
-        if (RB == 1) return NT;
+    auto lines = [&](int n, int RA, int RB) {
+        if (RB == 1) return nt;
         const int most = (64 * 1024 / int(sizeof(double2)) - n) / (n | 1);
-        return std::max(1, std::min(NT / std::max(RA, RB), most));
+        return std::max(1, std::min(nt / std::max(RA, RB), most));
     };
-    int L0 = std::min(lines(a.N0, a.RA0, a.RB0), a.N1);
-    if (L0 > 8 && L0 < a.N1) L0 = L0 / 8 * 8;
-    const int L1 = lines(a.N1, a.RA1, a.RB1);
-    const int nb0 = a.out[0] ? a.P * ((a.N1 + L0 - 1) / L0) : 0;
-    const int nb1 = a.out[1] ? int((long(a.P) * a.N0 + L1 - 1) / L1) : 0;
-    const size_t lds = sizeof(double2) * std::max(a.RB0 > 1 ? a.N0 + a.N0 * L0 : 0,
-                                                  a.RB1 > 1 ? a.N1 + (a.N1 | 1) * L1 : 0);
+    AxesShape s{nt, std::min(lines(a.N0, a.RA0, a.RB0), a.N1), lines(a.N1, a.RA1, a.RB1), 0};
+    if (s.L0 > 8 && s.L0 < a.N1) s.L0 = s.L0 / 8 * 8;
+    s.lds = sizeof(double2) * std::max(a.RB0 > 1 ? a.N0 + a.N0 * s.L0 : 0, a.RB1 > 1 ? a.N1 + (a.N1 | 1) * s.L1 : 0);
+    return s;
+}
+
+// Work-group size.  With at most kAxesFewGroups work-groups of one wave the
+// launch is latency and they are spread widest (us for 64, 128, 192, 256 threads:
+// 30 x 30, 4 planes 3.8, 4.1, 4.2, 4.3; 45 x 63, 21 planes 4.8, 5.0, 5.3, 5.6).
+// Otherwise the size that keeps most threads of a CU at work, given the waves its
+// registers allow, the LDS of the lines and the tasks these make, ties to the
+// smaller (120 x 120, 196 planes -, 30.6, 31.8, 33.5; 90 x 90, 64 planes -, 10.6,
+// 10.2, 9.4; 48 x 48, 2352 planes 44.5, 45.6, 47.1, 49.3), of those whose columns
+// fill 128-byte runs (one wave at 120 x 120: 5 columns, 44.9).
+constexpr long kAxesFewGroups = 1024;
+
+AxesShape axes_best_shape(const PlaneArgs& a)
+{
+    const AxesShape s1 = axes_shape(a, 64);
+    const long groups = long(a.P) * ((a.N1 + s1.L0 - 1) / s1.L0) + (long(a.P) * a.N0 + s1.L1 - 1) / s1.L1;
+    if (groups <= kAxesFewGroups) return s1;
+    const int waves = wide_radix(a) ? 12 : 16;  // of a CU
+    AxesShape best{};
+    long most = -1;
+    for (int nt = 64; nt <= kAxesMaxThreads; nt += 64) {
+        const AxesShape s = axes_shape(a, nt);
+        if (s.L0 < std::min(8, a.N1) && nt < kAxesMaxThreads) continue;
+        const long per_cu = std::min(waves * 64 / nt, s.lds ? int(kPlaneLds / s.lds) : 16);
+        const long busy = per_cu * (s.L0 * (a.RA0 + a.RB0) + s.L1 * (a.RA1 + a.RB1));
+        if (busy > most) {
+            most = busy;
+            best = s;
+        }
+    }
+    return best;
+}
+
+}  // namespace
+
+void launch_axes(const PlaneArgs& a, hipStream_t s)
+{
+    const AxesShape q = axes_best_shape(a);
+    const int nb0 = a.out[0] ? a.P * ((a.N1 + q.L0 - 1) / q.L0) : 0;
+    const int nb1 = a.out[1] ? int((long(a.P) * a.N0 + q.L1 - 1) / q.L1) : 0;
     if (wide_radix(a))
-        hipLaunchKernelGGL((axes_kernel<NT, 16>), dim3(nb0 + nb1), dim3(NT), lds, s, a, nb0, L0, L1);
+        hipLaunchKernelGGL(axes_kernel<16>, dim3(nb0 + nb1), dim3(q.nt), q.lds, s, a, nb0, q.L0, q.L1);
     else
-        hipLaunchKernelGGL((axes_kernel<NT, 12>), dim3(nb0 + nb1), dim3(NT), lds, s, a, nb0, L0, L1);
+        hipLaunchKernelGGL(axes_kernel<12>, dim3(nb0 + nb1), dim3(q.nt), q.lds, s, a, nb0, q.L0, q.L1);
 }
 
 void launch_plane_permute(const double* W, double* Wp, int P, int N0, int N1, hipStream_t s)

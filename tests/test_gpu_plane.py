@@ -75,6 +75,20 @@ def test_derivative_in_lds(model_dir):
         assert np.abs(eng.rhs(E, rho) - ref).max() <= 1e-11 * max(1.0, np.abs(ref).max())
 
 
+# 196 planes: one launch of work-groups of one wave (radices of at most 8), two,
+# three and four, with whole and ragged groups of columns and rows
+@pytest.mark.parametrize("grid", [(56, 35), (49, 30), (20, 120), (18, 100), (36, 60), (63, 45)])
+def test_derivative_work_groups(model_dir, grid):
+    p = _model("ipa14_hex120", model_dir, grid)
+    print("case", grid, flush=True)
+    o = oracle_py.Oracle(p)
+    eng = _engine(o, p)
+    rho = _rho(o, 10)
+    for E in _fields(o):
+        ref = o.rhs_E(E, rho)
+        assert np.abs(eng.rhs(E, rho) - ref).max() <= 1e-11 * max(1.0, np.abs(ref).max())
+
+
 @pytest.mark.parametrize("grid,layout", [((16, 16), FULL), ((3, 21), HERM), ((13, 33), HERM), ((30, 14), FULL),
                                          ((45, 22), FULL)])
 def test_exchange(model_dir, grid, layout):
