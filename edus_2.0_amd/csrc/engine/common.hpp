@@ -74,6 +74,14 @@ __device__ inline int xcd_contiguous_block()
     return x * q + min(x, r) + i;
 }
 
+// A table read at work-group-uniform indices by scalar loads: in device memory,
+// and not written while the kernel runs.
+typedef __attribute__((address_space(4))) double const_double;
+__device__ inline const const_double* uniform_doubles(const double* p)
+{
+    return reinterpret_cast<const const_double*>(reinterpret_cast<uintptr_t>(p));
+}
+
 // running maximum of a monitor: a NaN value becomes +inf, so it trips the
 // monitor instead of being dropped by fmax
 __device__ inline double mon_max(double m, double v) { return (v != v) ? __builtin_huge_val() : fmax(m, v); }

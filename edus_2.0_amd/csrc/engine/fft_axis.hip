@@ -285,10 +285,12 @@ __global__ void __launch_bounds__(NT) axis_fft_kernel(AxisFFTArgs a)
                 x[idx] = cmul(x[idx], ph);
             }
         } else if (a.mode == 0) {
+            const GroupCoef gc = group_coef(a.coef_tab, a.coef_stride, a.coef, a.P, a.ppi, a.axis == 1 ? row0 : plane0,
+                                            a.axis == 1 ? nlines : 1, a.axis == 1 ? a.N0 : 1);
             for (int idx = threadIdx.x; idx < nlines * n; idx += NT) {
                 const int c = idx / n;
                 const int j = idx - c * n;
-                const double coef = line_coef(a, a.axis == 1 ? (row0 + c) / a.N0 : plane0);
+                const double coef = gc.one ? gc.c : line_coef(a, a.axis == 1 ? (row0 + c) / a.N0 : plane0);
                 x[idx] = cmul_i(x[idx], coef * double(gamma_centred(j, n)));
             }
         } else {

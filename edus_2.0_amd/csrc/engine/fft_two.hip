@@ -139,6 +139,10 @@ __global__ void __launch_bounds__(NT) two_step_kernel(AxisFFTArgs a)
     constexpr int mode = MODE;
     constexpr bool sandwich = mode == 0 || mode == 3 || mode == 4 || mode == 5;
     constexpr bool deriv = mode == 0 || mode == 5;
+    GroupCoef gc{};
+    if constexpr (deriv)
+        gc = group_coef(a.coef_tab, a.coef_stride, a.coef, a.P, a.ppi, a.axis == 1 ? row0 : plane0,
+                        a.axis == 1 ? nlines : 1, a.axis == 1 ? a.N0 : 1);
 
     if constexpr (RB == 1) {
         // the whole line in one thread: no exchange
@@ -163,7 +167,7 @@ __global__ void __launch_bounds__(NT) two_step_kernel(AxisFFTArgs a)
                 });
             }
             if constexpr (deriv) {
-                const double coef = line_coef(a, a.axis == 1 ? (row0 + lineA) / a.N0 : plane0);
+                const double coef = gc.one ? gc.c : line_coef(a, a.axis == 1 ? (row0 + lineA) / a.N0 : plane0);
                 sfor<RA>([&](auto k_) {
                     constexpr int k = decltype(k_)::value;
                     v[k] = cmul_i(v[k], coef * double(gamma_centred(k, RA)));
@@ -281,7 +285,7 @@ __global__ void __launch_bounds__(NT) two_step_kernel(AxisFFTArgs a)
                         });
                     }
                     if constexpr (deriv) {
-                        const double coef = line_coef(a, a.axis == 1 ? (row0 + lineB) / a.N0 : plane0);
+                        const double coef = gc.one ? gc.c : line_coef(a, a.axis == 1 ? (row0 + lineB) / a.N0 : plane0);
                         sfor<RB>([&](auto k_) {
                             constexpr int k = decltype(k_)::value;
                             u[k] = cmul_i(u[k], coef * double(gamma_centred(ka + RA * k, n)));

@@ -79,8 +79,12 @@ __global__ void __launch_bounds__(kGradThreads) grad_fused_kernel(GradFusedArgs 
     const long plane = xcd_contiguous_block();
     const double2* in = a.in + plane * Nk;
     double2* out = a.out + plane * Nk;
-    const double c0 = a.coef_tab ? a.coef_tab[(plane / a.ppi) * a.coef_stride] : a.coef[0];
-    const double c1 = a.coef_tab ? a.coef_tab[(plane / a.ppi) * a.coef_stride + 1] : a.coef[1];
+    double c0 = a.coef[0], c1 = a.coef[1];
+    if (a.coef_tab) {
+        const const_double* t = uniform_doubles(a.coef_tab + (plane / a.ppi) * a.coef_stride);
+        c0 = t[0];
+        c1 = t[1];
+    }
     for (int i = tid; i < N0; i += kGradThreads) tw0[i] = a.tw0[i];
     for (int i = tid; i < N1; i += kGradThreads) tw1[i] = a.tw1[i];
 

@@ -142,6 +142,31 @@ __device__ inline double line_coef(const AxisFFTArgs& a, long plane)
     return a.coef_tab ? a.coef_tab[(plane / a.ppi) * a.coef_stride] : a.coef;
 }
 
+// Coefficient of a work-group's lines, formed at its start by scalar loads (a
+// load and a division per line in the middle of the transforms would be waited
+// for there): c when one is set, otherwise the lines are of several instances
+// and each looks its own up.  The lines are the `count` rows from row0 of planes
+// of `rows` rows (a group of columns: one row, its plane, with rows = 1), tab the
+// coefficient of instance 0 or null for c, P planes of ppi per instance.
+struct GroupCoef {
+    double c;
+    bool one;
+};
+__device__ inline GroupCoef group_coef(const double* tab, int stride, double c, int P, int ppi, long row0, int count,
+                                       int rows)
+{
+    if (!tab) return {c, true};
+    long inst = 0;
+    bool one = true;
+    if (P > ppi) {
+        const long plane = row0 / rows;
+        const int ahead = (int(row0 - plane * rows) + count - 1) / rows;  // planes after the first
+        inst = plane / ppi;
+        one = int(plane - inst * ppi) + ahead < ppi;
+    }
+    return {uniform_doubles(tab + inst * stride)[0], one};
+}
+
 // Axis-FFT tile configurations (threads per work-group, values per work-group)
 struct FFTConfig {
     int threads, values;

@@ -204,9 +204,12 @@ __global__ void __launch_bounds__(NT, MAXR <= 12 ? 4 : 2) plane_kernel(PlaneArgs
     bool both = true;
     double dl = 0.0, di = 0.0;  // derivative: coefficients of the outer and the inner axis
     if (!conv && !phase) {
-        const long inst = a.coef_tab ? plane / a.ppi : 0;
-        const double c0 = a.coef_tab ? a.coef_tab[inst * a.coef_stride] : a.coef[0];
-        const double c1 = a.coef_tab ? a.coef_tab[inst * a.coef_stride + 1] : a.coef[1];
+        double c0 = a.coef[0], c1 = a.coef[1];
+        if (a.coef_tab) {
+            const const_double* t = uniform_doubles(a.coef_tab + long(plane / a.ppi) * a.coef_stride);
+            c0 = t[0];
+            c1 = t[1];
+        }
         // (the same in every lane: kept in scalar registers)
         const bool use0 = __builtin_amdgcn_readfirstlane(c0 != 0.0), use1 = __builtin_amdgcn_readfirstlane(c1 != 0.0);
         if (!use0 && !use1) {
