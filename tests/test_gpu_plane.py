@@ -135,3 +135,25 @@ def test_batch_with_one_axis_members(model_dir):
         alone = e.get_state()
         batch.store(i)
         assert np.array_equal(e.get_state(), alone)
+
+
+def test_batch_of_two_pass_members(model_dir):
+    """As above where the axes are separate passes (240 x 180, above the field size
+    up to which such splits take one launch): groups of rows that hold the last
+    rows of one member and the first of the next."""
+    p = _model("ipa6_hex96", model_dir, (240, 180))
+    o = oracle_py.Oracle(p)
+    engines = [_engine(o, p) for _ in range(3)]
+    E = np.zeros((4, 3, 3, 3))
+    rng = np.random.default_rng(7)
+    for i, e in enumerate(_fields(o)):
+        E[:, :, i, :] = rng.uniform(0.5, 1.0, (4, 3, 1)) * np.array(e)
+    for e in engines:
+        e.set_state(o.rho + 0.05 * _rho(o, 8))
+    batch = edus.Batch(engines)
+    batch.rk4_steps(0.05, E)
+    for i, e in enumerate(engines):
+        e.rk4_steps(0.05, E[:, :, i])
+        alone = e.get_state()
+        batch.store(i)
+        assert np.array_equal(e.get_state(), alone)
