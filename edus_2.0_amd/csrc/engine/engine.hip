@@ -790,16 +790,24 @@ void Engine::autotune()
             HIP_CHECK(hipEventCreate(&e1));
             const double cg[2] = {1e-3, 1e-3};
             CommArgs c = tuning_stage_args(comm_kind);
+            // with exchange the derivative alone: T and W are not allocated yet, and
+            // on these grids the exchange term's passes are the same in either form
+            auto derivative = [&] {
+                c.D = c.D2 = nullptr;
+                if (coulomb)
+                    c.D = gradient(c.rho, cg, nullptr, true, true);
+                else
+                    derivative_terms(c, cg, nullptr, nullptr, nullptr, true, true);
+            };
             float best[2] = {1e30f, 1e30f};
             for (int trial = 0; trial < 3; ++trial)
                 for (int f = 0; f < 2; ++f) {
                     grad_fused = f == 1;
-                    c.D = c.D2 = nullptr;
-                    derivative_terms(c, cg, nullptr, nullptr, nullptr, true, true);  // warm-up
+                    derivative();  // warm-up
                     launch_comm(nb, layout, comm_kind, comm_tile, c, s);
                     HIP_CHECK(hipEventRecord(e0, s));
                     for (int r = 0; r < 8; ++r) {
-                        derivative_terms(c, cg, nullptr, nullptr, nullptr, true, true);
+                        derivative();
                         launch_comm(nb, layout, comm_kind, comm_tile, c, s);
                     }
                     HIP_CHECK(hipEventRecord(e1, s));
@@ -1018,6 +1026,7 @@ const double2* Engine::kgradient(const double2* in, const double E[3], const dou
 // term costs no pass of its own.
 void Engine::fock(const double2* in, bool row_done)
 {
+    if (!T || !W || !hsum) throw EngineError(EDUS_ERR_STATE, "exchange term before its arrays are set up");
     if (plane_exchange()) {
         plane_launch(in, false, nullptr, nullptr, true);
         return;
