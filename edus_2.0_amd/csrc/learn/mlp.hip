@@ -270,8 +270,10 @@ int cdiv(long a, long b) { return int((a + b - 1) / b); }
 void launch_gemm(const GemmArgs& g, int nz, hipStream_t s)
 {
     const dim3 grid(cdiv(g.M, kTile), cdiv(g.N, kTile), nz);
-    const bool ak = g.sak == 1;
-    if (g.sbn != 1 || (!ak && g.sam != 1) || (ak && g.ones_row >= 0))
+    // (a layer of one input has both strides 1: its weight gradient, with the row
+    // of ones, is the form with contiguous rows)
+    const bool ak = g.sak == 1 && g.ones_row < 0;
+    if (g.sbn != 1 || (!ak && g.sam != 1))
         throw EngineError(EDUS_ERR_ARG, "GEMM operand order not supported");
     // 8-byte loads where every row starts on 8 bytes; kchunk is a multiple of 16
     const long ld = ak ? g.sam : g.sak;
