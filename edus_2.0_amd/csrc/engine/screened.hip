@@ -46,7 +46,6 @@
 // of bands, r multiplied instead of divided), so results agree to rounding,
 // not bit for bit.
 #include <algorithm>
-#include <atomic>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -692,11 +691,13 @@ __global__ void __launch_bounds__(256) lindhard_sum_kernel(LindhardMfmaArgs a)
 }
 
 constexpr int kLindMaxUPW = 3;
+constexpr size_t kLindMfmaLds = 160 * 1024;
 
-// The shape of the matrix-core form, and whether it is used.  Among the window
-// lengths GT that fit, and 1 to 3 parts of the k range, the one with the least
-// estimated time: rounds of resident work-groups x steps x the longer of a
-// step's FP64 issue time on a SIMD and its latency.
+// The shape of the matrix-core form, and whether it is used: functions of the
+// sizes alone, so that a call under stream capture runs the kernels that it runs
+// elsewhere.  Among the window lengths GT that fit, and 1 to 3 parts of the k
+// range, the one with the least estimated time: rounds of resident work-groups x
+// steps x the longer of a step's FP64 issue time on a SIMD and its latency.
 //
 // The vector form is left the shapes it does better: two bands, where 3 of 16
 // columns would be used, and, where it fills the chip with four q per lane
@@ -724,7 +725,7 @@ bool lindhard_mfma_shape(const LindhardPlan& p, LindhardMfmaArgs& best)
         const LindhardMfmaLds sz(nv, nc, T, GT);
         const size_t lds = size_t(sz.elems(GT)) * sizeof(double2);
         const int units = (GT / 4) * T, upw = (units + W - 1) / W;
-        if (lds > 160 * 1024 || upw > kLindMaxUPW || GT * nc * nv > 2 * nt) continue;
+        if (lds > kLindMfmaLds || upw > kLindMaxUPW || GT * nc * nv > 2 * nt) continue;
         const int per_cu = std::max(1, std::min(int(160 * 1024 / lds), 12 / W));
         const int blocks = N0 * ((N1 + GT - 1) / GT);
         for (int KS = 1; KS <= 3; ++KS) {
@@ -758,55 +759,46 @@ bool lindhard_mfma_shape(const LindhardPlan& p, LindhardMfmaArgs& best)
     return true;
 }
 
-// false: not launched.  More than 64 KB of LDS needs the kernel's limit raised,
-// which does not reach a launch that is being captured: a first call under
-// capture is left to the vector form.
 template <int CV, int CC, int UPW>
-bool launch_mfma_one(const LindhardMfmaArgs& a, hipStream_t s)
+void launch_mfma_one(const LindhardMfmaArgs& a, hipStream_t s)
 {
     const size_t lds = size_t(LindhardMfmaLds(a.nv, a.nc, a.T, a.GT).elems(a.GT)) * sizeof(double2);
     auto kern = &lindhard_mfma_kernel<CV, CC, UPW>;
-    static std::atomic<bool> raised{false};  // calls may come from several host threads
-    if (lds > 64 * 1024 && !raised.load()) {
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        if (s) EDUS_HIP_CHECK(hipStreamIsCapturing(s, &st));
-        if (st != hipStreamCaptureStatusNone) return false;
+    // a first call may be under stream capture: the launch captured there runs with
+    // its LDS all the same (checked by replays of 80 KB launches)
+    static std::once_flag raised;  // calls may come from several host threads
+    std::call_once(raised, [&] {
         EDUS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-        raised.store(true);
-    }
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, int(kLindMfmaLds)));
+    });
     hipLaunchKernelGGL(kern, dim3(a.N0 * a.nqb_row * a.KS), dim3(lind_threads(CV, CC)), lds, s, a);
-    return true;
 }
 
 template <int CV, int CC>
-bool launch_mfma_upw(const LindhardMfmaArgs& a, hipStream_t s)
+void launch_mfma_upw(const LindhardMfmaArgs& a, hipStream_t s)
 {
     const int W = lind_threads(CV, CC) / 64;
     switch (((a.GT / 4) * a.T + W - 1) / W) {
-        case 1: return launch_mfma_one<CV, CC, 1>(a, s);
-        case 2: return launch_mfma_one<CV, CC, 2>(a, s);
-        default: return launch_mfma_one<CV, CC, kLindMaxUPW>(a, s);
+        case 1: launch_mfma_one<CV, CC, 1>(a, s); break;
+        case 2: launch_mfma_one<CV, CC, 2>(a, s); break;
+        default: launch_mfma_one<CV, CC, kLindMaxUPW>(a, s); break;
     }
 }
 
-bool launch_lindhard_mfma(const LindhardMfmaArgs& a, hipStream_t s)
+void launch_lindhard_mfma(const LindhardMfmaArgs& a, hipStream_t s)
 {
-    bool done = false;
     switch ((a.nv + 3) / 4 * 8 + (a.nc + 3) / 4) {
 #define EDUS_CVCC(cv, cc) \
-    case cv * 8 + cc: done = launch_mfma_upw<cv, cc>(a, s); break;
+    case cv * 8 + cc: launch_mfma_upw<cv, cc>(a, s); break;
         EDUS_CVCC(1, 1) EDUS_CVCC(1, 2) EDUS_CVCC(1, 3) EDUS_CVCC(1, 4) EDUS_CVCC(2, 1) EDUS_CVCC(2, 2)
         EDUS_CVCC(2, 3) EDUS_CVCC(3, 1) EDUS_CVCC(3, 2) EDUS_CVCC(4, 1)
 #undef EDUS_CVCC
         default: break;
     }
-    if (!done) return false;
     if (a.KS > 1)
         hipLaunchKernelGGL(lindhard_sum_kernel, dim3((a.Nk + kLindSumQ - 1) / kLindSumQ), dim3(256),
                            size_t(a.P) * kLindSumQ * sizeof(double2), s, a);
     EDUS_HIP_CHECK(hipGetLastError());
-    return true;
 }
 
 // waves per q for L element pairs (fractional when several q share a wave)
@@ -878,7 +870,8 @@ void launch_lindhard(const LindhardPlan& p, const double2* U, const double* eps,
         m.eps = eps;
         m.X = X;
         m.work = work;
-        if (launch_lindhard_mfma(m, s)) return;
+        launch_lindhard_mfma(m, s);
+        return;
     }
     double2* Uv = work;
     double2* Uc = work + size_t(p.Nk) * p.nv * p.nb;
