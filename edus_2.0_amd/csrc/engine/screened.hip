@@ -434,20 +434,26 @@ struct LindhardMfmaLds {
     __host__ __device__ int elems(int GT) const { return (GT + 1) * ring + 2 * A + (2 * r + 1) / 2; }
 };
 
-// Threads, and products A_v (n = CV) or B_c (n = CC) per thread and step, by the
-// numbers of valence and conduction quadruples, nb <= 4 (CV + CC) and nb <= 16
+// By the numbers of valence and conduction quadruples, for at most NB (8 or 12)
+// bands: threads, and products A_v (n = CV) or B_c (n = CC) per thread and step
 constexpr int lind_threads(int CV, int CC) { return CV + CC <= 3 ? 256 : 512; }
-// (at most 16 * 17 / 2 pairs times 4 n bands, n quadruples)
-constexpr int lind_items(int n, int CV, int CC)
+constexpr int lind_items(int n, int CV, int CC, int NB)
 {
-    const int nb = 4 * (CV + CC) < 16 ? 4 * (CV + CC) : 16, bands = 4 * n < nb ? 4 * n : nb - 1;
+    const int nb = 4 * (CV + CC) < NB ? 4 * (CV + CC) : NB, bands = 4 * n < nb ? 4 * n : nb - 1;
     return (nb * (nb + 1) / 2 * bands + lind_threads(CV, CC) - 1) / lind_threads(CV, CC);
 }
+// Waves per SIMD that the registers leave (116 to 166 at NB = 8, up to 217 at 12).
+// Lists sized for 12 bands and a choice of shapes that counted on three waves: 6
+// bands, 1 filled, 52 x 52 2362 us; with lists for 8 bands 1538; vector form 1357.
+constexpr int lind_waves(int NB) { return NB <= 8 ? 3 : 2; }
+// the same as a limit for the compiler (two conduction quadruples: 163 without the
+// limit, with it some spill)
+constexpr int lind_min_waves(int CC, int NB) { return CC == 2 ? 2 : lind_waves(NB); }
 
-template <int CV, int CC, int UPW>
-__global__ void __launch_bounds__(lind_threads(CV, CC)) lindhard_mfma_kernel(LindhardMfmaArgs a)
+template <int CV, int CC, int UPW, int NBANDS>
+__global__ void __launch_bounds__(lind_threads(CV, CC), (lind_min_waves(CC, NBANDS))) lindhard_mfma_kernel(LindhardMfmaArgs a)
 {
-    constexpr int NT = lind_threads(CV, CC), NA = lind_items(CV, CV, CC), NB = lind_items(CC, CV, CC);
+    constexpr int NT = lind_threads(CV, CC), NA = lind_items(CV, CV, CC, NBANDS), NB = lind_items(CC, CV, CC, NBANDS);
     extern __shared__ double2 lds[];
     const int nb = a.nb, nv = a.nv, nc = a.nc, N0 = a.N0, N1 = a.N1, P = a.P, T = a.T, GT = a.GT;
     const int Pp = 16 * T;
@@ -693,40 +699,61 @@ __global__ void __launch_bounds__(256) lindhard_sum_kernel(LindhardMfmaArgs a)
 constexpr int kLindMaxUPW = 3;
 constexpr size_t kLindMfmaLds = 160 * 1024;
 
+// Whether the vector form is the faster one.  How full it runs the chip goes by
+// its waves (one or more per q-block): 4 to 6 per CU in one round are its best
+// case, a second round just started its worst; with four q per lane (TQ = 4) any
+// large grid fills it.  The matrix form pads the bands of either side to
+// quadruples: with one quadruple each it was the faster one at every size, with
+// two on one side up to half of its products are padding, and with two on both, or
+// 13 bands and more, its registers hold fewer waves than its latency needs.  us,
+// vector and matrix form (waves of the vector form):
+//   3, 1 filled   64 x 64 (448): 1327, 1168; 72 x 72 (576): 1906, 2153
+//   4, 2          56 x 56 (560): 1300, 898; 72 x 72 (864): 2151, 2191
+//   6, 3          72 x 72: 3293, 2922        8, 4   48 x 48: 2800, 971
+//   6, 5          48 x 48 (768): 922, 921; 52 x 52 (936): 1076, 1385
+//   7, 6          48 x 48 (1152): 1106, 925; 52 x 52 (1352): 1309, 1417
+//   8, 1          40 x 40 (1600): 1171, 1169; 48 x 48 (2304): 2085, 2200
+//   8, 2          42 x 42 (1764): 1411, 1180; 45 x 45 (2025): 1637, 2016; 52 x 52 (2704): 3726, 2518
+//   8, 7          32 x 32 (1024): 448, 406; 45 x 26 (1170): 599, 683; 40 x 40 (1600): 1384, 977
+//   10, 5         48 x 48: 3582, 3672
+//   11, 8         36 x 21 (1512): 533, 576; 28 x 28 (1568): 894, 670; 44 x 44 (3872): 1.31 times
+//   12, 11        22 x 18 (792): 241, 282; 45 x 26 (2340): 1.09 times; 42 x 42 (3528): 1.44 times
+//   13, 12        24 x 24: 393, 370; 26 x 26: 455, 635
+//   14, 5         30 x 30: 1177, 2133        14, 13   40 x 40: 2690, 5432
+bool lindhard_vector_better(const LindhardPlan& p)
+{
+    const int nb = p.nb, nv = p.nv, nc = p.nc;
+    const long waves = long(p.blocks) * p.W;
+    if (nb < 3 || nb > 12) return true;
+    if (nb > 8) return nb <= 10 || nc > 4 || p.TQ != 1 || waves < 1536;
+    if (nb <= 4) return p.TQ != 1 || waves >= (nb == 3 ? 512 : 1024);
+    if (nv <= 4 && nc <= 4) return false;
+    if (p.TQ != 1) return true;
+    if (nb == 6) return waves >= 900;
+    if (nb == 7) return nc == 1 && waves >= 1300;
+    if (nv == 1) return true;
+    if (nv == 2) return waves >= 1900 && waves < 2400;
+    return nc <= 2 && waves >= 1100 && waves < 1560;
+}
+
 // The shape of the matrix-core form, and whether it is used: functions of the
 // sizes alone, so that a call under stream capture runs the kernels that it runs
 // elsewhere.  Among the window lengths GT that fit, and 1 to 3 parts of the k
 // range, the one with the least estimated time: rounds of resident work-groups x
 // steps x the longer of a step's FP64 issue time on a SIMD and its latency.
-//
-// The vector form is left the shapes it does better: two bands, where 3 of 16
-// columns would be used, and, where it fills the chip with four q per lane
-// (TQ = 4) or enough waves, those with more than one quadruple to pad.  us,
-// vector and matrix form: 3 bands, 1 filled, 40 x 40: 980, 487 (120 x 120: 6055,
-// 10315); 6, 3, 96 x 96: 9842, 7218; 8, 4, 48 x 48: 3003, 1235, 90 x 90: 22890,
-// 13998; 8, 7, 48 x 48: 2421, 1427 (96 x 96: 13263, 28374); 10, 5, 48 x 48: 3582,
-// 3672; 12, 6, 40 x 40: 3335, 2896; 14, 7, 30 x 30: 1569, 1352 (48 x 48: 6902, 10052).
 bool lindhard_mfma_shape(const LindhardPlan& p, LindhardMfmaArgs& best)
 {
     const int nb = p.nb, nv = p.nv, nc = p.nc, N0 = p.N0, N1 = p.N1;
-    if (nv < 1 || nc < 1 || nb < 3) return false;
+    if (nv < 1 || nc < 1 || lindhard_vector_better(p)) return false;
     const int P = nb * (nb + 1) / 2, T = (P + 15) / 16, CV = (nv + 3) / 4, CC = (nc + 3) / 4;
-    const bool small = p.TQ == 1;
-    if (nb <= 4) {
-        if (!small || long(p.blocks) * p.W >= 1024) return false;
-    } else if (nb <= 8) {
-        if (!(CV == 1 && CC == 1) && (!small || (nb == 8 && nv == 1))) return false;
-    } else if (!small || nb <= 10) {
-        return false;
-    }
-    const int nt = lind_threads(CV, CC), W = nt / 64;
+    const int nt = lind_threads(CV, CC), W = nt / 64, simd_waves = lind_waves(nb);
     double best_cost = 1e300;
     for (int GT = 4; GT <= 32; GT += 4) {
         const LindhardMfmaLds sz(nv, nc, T, GT);
         const size_t lds = size_t(sz.elems(GT)) * sizeof(double2);
         const int units = (GT / 4) * T, upw = (units + W - 1) / W;
         if (lds > kLindMfmaLds || upw > kLindMaxUPW || GT * nc * nv > 2 * nt) continue;
-        const int per_cu = std::max(1, std::min(int(160 * 1024 / lds), 12 / W));
+        const int per_cu = std::max(1, std::min(int(kLindMfmaLds / lds), 4 * simd_waves / W));
         const int blocks = N0 * ((N1 + GT - 1) / GT);
         for (int KS = 1; KS <= 3; ++KS) {
             if (KS > 1 && N0 < 4 * KS) continue;
@@ -759,11 +786,11 @@ bool lindhard_mfma_shape(const LindhardPlan& p, LindhardMfmaArgs& best)
     return true;
 }
 
-template <int CV, int CC, int UPW>
+template <int CV, int CC, int UPW, int NB>
 void launch_mfma_one(const LindhardMfmaArgs& a, hipStream_t s)
 {
     const size_t lds = size_t(LindhardMfmaLds(a.nv, a.nc, a.T, a.GT).elems(a.GT)) * sizeof(double2);
-    auto kern = &lindhard_mfma_kernel<CV, CC, UPW>;
+    auto kern = &lindhard_mfma_kernel<CV, CC, UPW, NB>;
     // a first call may be under stream capture: the launch captured there runs with
     // its LDS all the same (checked by replays of 80 KB launches)
     static std::once_flag raised;  // calls may come from several host threads
@@ -774,26 +801,26 @@ void launch_mfma_one(const LindhardMfmaArgs& a, hipStream_t s)
     hipLaunchKernelGGL(kern, dim3(a.N0 * a.nqb_row * a.KS), dim3(lind_threads(CV, CC)), lds, s, a);
 }
 
-template <int CV, int CC>
+template <int CV, int CC, int NB>
 void launch_mfma_upw(const LindhardMfmaArgs& a, hipStream_t s)
 {
     const int W = lind_threads(CV, CC) / 64;
     switch (((a.GT / 4) * a.T + W - 1) / W) {
-        case 1: launch_mfma_one<CV, CC, 1>(a, s); break;
-        case 2: launch_mfma_one<CV, CC, 2>(a, s); break;
-        default: launch_mfma_one<CV, CC, kLindMaxUPW>(a, s); break;
+        case 1: launch_mfma_one<CV, CC, 1, NB>(a, s); break;
+        case 2: launch_mfma_one<CV, CC, 2, NB>(a, s); break;
+        default: launch_mfma_one<CV, CC, kLindMaxUPW, NB>(a, s); break;
     }
 }
 
 void launch_lindhard_mfma(const LindhardMfmaArgs& a, hipStream_t s)
 {
-    switch ((a.nv + 3) / 4 * 8 + (a.nc + 3) / 4) {
-#define EDUS_CVCC(cv, cc) \
-    case cv * 8 + cc: launch_mfma_upw<cv, cc>(a, s); break;
-        EDUS_CVCC(1, 1) EDUS_CVCC(1, 2) EDUS_CVCC(1, 3) EDUS_CVCC(1, 4) EDUS_CVCC(2, 1) EDUS_CVCC(2, 2)
-        EDUS_CVCC(2, 3) EDUS_CVCC(3, 1) EDUS_CVCC(3, 2) EDUS_CVCC(4, 1)
-#undef EDUS_CVCC
-        default: break;
+    switch ((a.nb > 8 ? 64 : 0) + (a.nv + 3) / 4 * 8 + (a.nc + 3) / 4) {  // (those lindhard_vector_better leaves)
+        case 1 * 8 + 1: launch_mfma_upw<1, 1, 8>(a, s); break;
+        case 1 * 8 + 2: launch_mfma_upw<1, 2, 8>(a, s); break;
+        case 2 * 8 + 1: launch_mfma_upw<2, 1, 8>(a, s); break;
+        case 64 + 2 * 8 + 1: launch_mfma_upw<2, 1, 12>(a, s); break;
+        case 64 + 3 * 8 + 1: launch_mfma_upw<3, 1, 12>(a, s); break;
+        default: throw EngineError(EDUS_ERR_STATE, "lindhard: no matrix-core kernel for these bands");
     }
     if (a.KS > 1)
         hipLaunchKernelGGL(lindhard_sum_kernel, dim3((a.Nk + kLindSumQ - 1) / kLindSumQ), dim3(256),
