@@ -113,10 +113,12 @@ std::map<CommKey, std::tuple<int, int, int>>& tuned_comm()
     return m;
 }
 
-// one-pass gradient or not per (N0, N1, planes of all instances)
-std::map<std::tuple<int, int, int>, bool>& tuned_grad()
+// one-pass gradient or not per (N0, N1, nb, layout, precision, exchange,
+// upper-triangle fields): all that the timed stage depends on
+using GradKey = std::tuple<int, int, int, int, int, int, int>;
+std::map<GradKey, bool>& tuned_grad()
 {
-    static std::map<std::tuple<int, int, int>, bool> m;
+    static std::map<GradKey, bool> m;
     return m;
 }
 
@@ -681,148 +683,24 @@ void Engine::autotune()
         tuned_shapes()[key] = best_c;
     }
 
-    // commutator engine and tile, whichever is fastest here: for FP64 the FMA
-    // engine or the matrix cores (they differ in summation order only), for
-    // mixed precision the FP32 matrix cores; tiles give identical results.
-    // The Adams-Bashforth kernel (history prefetched, more registers) gets a
-    // tile of its own.
-    const CommKey ckey = std::make_tuple(nb, layout, Nk * B, prec, force_kind, int(coulomb), int(tri),
-                                         kgrad ? (stencil_fused() ? 2 : 0) : int(axes_together()));
-    auto cit = tuned_comm().find(ckey);
-    if (cit != tuned_comm().end()) {
-        comm_kind = std::get<0>(cit->second);
-        comm_tile = std::get<1>(cit->second);
-        comm_tile_ab = std::get<2>(cit->second);
-    } else {
-        std::vector<std::pair<int, int>> cands;
-        if (prec == EDUS_PREC_MIXED)
-            cands = {{kCommMfma32, 0}, {kCommMfma32, 1}, {kCommMfma32, 2}};
-        else
-            cands = {{kCommScalar, 0}, {kCommMfma64, 0}, {kCommMfma64, 1}, {kCommMfma64, 2}};
-        if (force_kind >= 0) {  // keep the members' engine: only the tile is free
-            std::vector<std::pair<int, int>> keep;
-            for (const auto& kt : cands)
-                if (kt.first == force_kind) keep.push_back(kt);
-            cands = keep.empty() ? std::vector<std::pair<int, int>>{{force_kind, 0}} : keep;
-        }
-        hipEvent_t e0, e1;
-        HIP_CHECK(hipEventCreate(&e0));
-        HIP_CHECK(hipEventCreate(&e1));
-        auto time_of = [&](int kind, int tile, const CommArgs& c) {
-            // with the stage's set, and for RK4 the other stages': one array read
-            // and written beside the operands
-            CommArgs lite = c;
-            if (!c.up.ab_order) lite.up.out1 = nullptr;
-            auto step = [&] {
-                for (int r = 0; r < 4; ++r) launch_comm(nb, layout, kind, tile, r == 2 ? c : lite, s);
-            };
-            step();  // warm-up
-            HIP_CHECK(hipEventRecord(e0, s));
-            step();
-            step();
-            HIP_CHECK(hipEventRecord(e1, s));
-            HIP_CHECK(hipEventSynchronize(e1));
-            float ms = 0.f;
-            HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-            return ms;
-        };
-        // the operand sets of the hot uses, so that the candidates see the
-        // step's real HBM traffic, not a cache-resident subset.
-        // Adams-Bashforth step of order 4: state (read and written in place),
-        // H0, one xi, D and three history arrays read, the new history entry
-        // written (over one of them: each element is read and written by the
-        // same thread)
-        auto ab_args = [&](int kind) {
-            CommArgs cab = tuning_stage_args(kind);
-            cab.up = StageUpdate{};
-            if (cab.nst > 0) {  // an Adams-Bashforth step updates the state in place: a stencil pass of its own
-                cab.nst = 0;
-                cab.D = D;
-            }
-            if (cab.D2) cab.D2 = f;
-            cab.up.ab_order = 4;
-            cab.up.y = aux;
-            cab.up.out_f = G;
-            cab.up.hist[1] = acc;
-            cab.up.hist[2] = G;
-            cab.up.hist[3] = f;
-            return cab;
-        };
-        float best = 1e30f;
-        for (const auto& kt : cands) {
-            const float ms = time_of(kt.first, kt.second, tuning_stage_args(kt.first));
-            if (ms < best) {
-                best = ms;
-                comm_kind = kt.first;
-                comm_tile = kt.second;
-            }
-        }
-        best = 1e30f;
-        for (const auto& kt : cands) {
-            if (kt.first != comm_kind) continue;
-            const float ms = time_of(kt.first, kt.second, ab_args(kt.first));
-            if (ms < best) {
-                best = ms;
-                comm_tile_ab = kt.second;
-            }
-        }
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
-        HIP_CHECK(hipGetLastError());
-        tuned_comm()[ckey] = std::make_tuple(comm_kind, comm_tile, comm_tile_ab);
-    }
-    // the spectral derivative: one pass per plane or two axis passes, whichever
-    // gives the faster stage (timed with the commutator that consumes D: the
-    // one-pass form leaves different data in the caches); they agree to rounding
+    // the spectral derivative: one pass per plane or axis passes.  Decided before
+    // the commutator is tuned, whose operands depend on it
     grad_fused = false;
-    if (grad_form_choice(N0, N1) && plane_ok && coulomb && !kgrad) {
-        grad_fused = force_grad != 0;  // derivative and exchange term in one launch
-    } else if (grad_form_choice(N0, N1) && !kgrad) {
-        const auto gkey = std::make_tuple(N0, N1, B * npl);
-        auto git = tuned_grad().find(gkey);
-        if (force_grad >= 0) {  // a batch group keeps its members' form (they differ in rounding)
-            grad_fused = force_grad == 1;
-        } else if (git != tuned_grad().end()) {
-            grad_fused = git->second;
-        } else {
-            hipEvent_t e0, e1;
-            HIP_CHECK(hipEventCreate(&e0));
-            HIP_CHECK(hipEventCreate(&e1));
-            const double cg[2] = {1e-3, 1e-3};
-            CommArgs c = tuning_stage_args(comm_kind);
-            // with exchange the derivative alone: T and W are not allocated yet, and
-            // on these grids the exchange term's passes are the same in either form
-            auto derivative = [&] {
-                c.D = c.D2 = nullptr;
-                if (coulomb)
-                    c.D = gradient(c.rho, cg, nullptr, true, true);
-                else
-                    derivative_terms(c, cg, nullptr, nullptr, nullptr, true, true);
-            };
-            float best[2] = {1e30f, 1e30f};
-            for (int trial = 0; trial < 3; ++trial)
-                for (int f = 0; f < 2; ++f) {
-                    grad_fused = f == 1;
-                    derivative();  // warm-up
-                    launch_comm(nb, layout, comm_kind, comm_tile, c, s);
-                    HIP_CHECK(hipEventRecord(e0, s));
-                    for (int r = 0; r < 8; ++r) {
-                        derivative();
-                        launch_comm(nb, layout, comm_kind, comm_tile, c, s);
-                    }
-                    HIP_CHECK(hipEventRecord(e1, s));
-                    HIP_CHECK(hipEventSynchronize(e1));
-                    float ms = 0.f;
-                    HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-                    best[f] = std::min(best[f], ms);
-                }
-            (void)hipEventDestroy(e0);
-            (void)hipEventDestroy(e1);
-            HIP_CHECK(hipGetLastError());
-            grad_fused = best[1] < 0.98f * best[0];  // the two passes unless the other form is clearly faster
-            tuned_grad()[gkey] = grad_fused;
-        }
+    if (grad_form_choice(N0, N1) && !kgrad) {
+        if (coulomb && plane_ok)
+            grad_fused = force_grad != 0;  // derivative and exchange term in one launch
+        else if (force_grad >= 0)
+            grad_fused = force_grad == 1;  // a batch group keeps its members' form (they differ in rounding)
+        else if (peierls)
+            // no derivative there: the phase's form, whose one-pass kernel wants planes
+            // for half the CUs (us for ten steps, two passes and one, 90 x 90: 81 planes
+            // 1020, 1036; 100 planes 1174, 1162; 196 planes 1738, 1604; 96 x 96: 64 planes
+            // 954, 1003; 100 planes 1386, 1310; 196 planes 1936, 1730)
+            grad_fused = plane_form(N0, N1) && npl >= 96;
+        else
+            tune_gradient();
     }
+    tune_commutator();
 
     if (prec == EDUS_PREC_MIXED) {
         // set-up products (the velocity operator) stay FP64
@@ -836,6 +714,166 @@ void Engine::autotune()
     for (double2* p : {G, f, acc, aux}) HIP_CHECK(hipMemsetAsync(p, 0, plane_bytes(), s));
     HIP_CHECK(hipStreamSynchronize(s));
     prime_launch_attributes();
+}
+
+// Commutator engine and tile, whichever is fastest here: for FP64 the FMA
+// engine or the matrix cores (they differ in summation order only), for
+// mixed precision the FP32 matrix cores; tiles give identical results.
+// The Adams-Bashforth kernel (history prefetched, more registers) gets a
+// tile of its own.
+void Engine::tune_commutator()
+{
+    const CommKey ckey = std::make_tuple(nb, layout, Nk * B, prec, force_kind, int(coulomb), int(tri),
+                                         kgrad ? (stencil_fused() ? 2 : 0) : int(axes_together()));
+    auto cit = tuned_comm().find(ckey);
+    if (cit != tuned_comm().end()) {
+        comm_kind = std::get<0>(cit->second);
+        comm_tile = std::get<1>(cit->second);
+        comm_tile_ab = std::get<2>(cit->second);
+        return;
+    }
+    std::vector<std::pair<int, int>> cands;
+    if (prec == EDUS_PREC_MIXED)
+        cands = {{kCommMfma32, 0}, {kCommMfma32, 1}, {kCommMfma32, 2}};
+    else
+        cands = {{kCommScalar, 0}, {kCommMfma64, 0}, {kCommMfma64, 1}, {kCommMfma64, 2}};
+    if (force_kind >= 0) {  // keep the members' engine: only the tile is free
+        std::vector<std::pair<int, int>> keep;
+        for (const auto& kt : cands)
+            if (kt.first == force_kind) keep.push_back(kt);
+        cands = keep.empty() ? std::vector<std::pair<int, int>>{{force_kind, 0}} : keep;
+    }
+    hipEvent_t e0, e1;
+    HIP_CHECK(hipEventCreate(&e0));
+    HIP_CHECK(hipEventCreate(&e1));
+    auto time_of = [&](int kind, int tile, const CommArgs& c) {
+        // with the stage's set, and for RK4 the other stages': one array read
+        // and written beside the operands
+        CommArgs lite = c;
+        if (!c.up.ab_order) lite.up.out1 = nullptr;
+        auto step = [&] {
+            for (int r = 0; r < 4; ++r) launch_comm(nb, layout, kind, tile, r == 2 ? c : lite, s);
+        };
+        step();  // warm-up
+        HIP_CHECK(hipEventRecord(e0, s));
+        step();
+        step();
+        HIP_CHECK(hipEventRecord(e1, s));
+        HIP_CHECK(hipEventSynchronize(e1));
+        float ms = 0.f;
+        HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
+        return ms;
+    };
+    // the operand sets of the hot uses, so that the candidates see the
+    // step's real HBM traffic, not a cache-resident subset.
+    // Adams-Bashforth step of order 4: state (read and written in place),
+    // H0, one xi, D and three history arrays read, the new history entry
+    // written (over one of them: each element is read and written by the
+    // same thread)
+    auto ab_args = [&](int kind) {
+        CommArgs cab = tuning_stage_args(kind);
+        cab.up = StageUpdate{};
+        if (cab.nst > 0) {  // an Adams-Bashforth step updates the state in place: a stencil pass of its own
+            cab.nst = 0;
+            cab.D = D;
+        }
+        if (cab.D2) cab.D2 = f;
+        cab.up.ab_order = 4;
+        cab.up.y = aux;
+        cab.up.out_f = G;
+        cab.up.hist[1] = acc;
+        cab.up.hist[2] = G;
+        cab.up.hist[3] = f;
+        return cab;
+    };
+    float best = 1e30f;
+    for (const auto& kt : cands) {
+        const float ms = time_of(kt.first, kt.second, tuning_stage_args(kt.first));
+        if (ms < best) {
+            best = ms;
+            comm_kind = kt.first;
+            comm_tile = kt.second;
+        }
+    }
+    best = 1e30f;
+    for (const auto& kt : cands) {
+        if (kt.first != comm_kind) continue;
+        const float ms = time_of(kt.first, kt.second, ab_args(kt.first));
+        if (ms < best) {
+            best = ms;
+            comm_tile_ab = kt.second;
+        }
+    }
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    HIP_CHECK(hipGetLastError());
+    tuned_comm()[ckey] = std::make_tuple(comm_kind, comm_tile, comm_tile_ab);
+}
+
+// The spectral derivative in one pass per plane or in axis passes, whichever
+// gives the faster step (timed with the commutator that consumes D: the
+// one-pass form leaves different data in the caches); they agree to rounding.
+// For one instance (a batch group takes its members' form).
+void Engine::tune_gradient()
+{
+    const GradKey gkey = std::make_tuple(N0, N1, nb, layout, prec, int(coulomb), int(tri));
+    auto git = tuned_grad().find(gkey);
+    if (git != tuned_grad().end()) {
+        grad_fused = git->second;
+        return;
+    }
+    // the commutator's choice for either form
+    int kind[2], tile[2];
+    for (int f = 0; f < 2; ++f) {
+        grad_fused = f == 1;
+        tune_commutator();
+        kind[f] = comm_kind;
+        tile[f] = comm_tile;
+    }
+    // an RK4 step of length 0 on the arrays of a real one (at 14 bands on 120 x 120
+    // these are about the size of the cache behind HBM, and a single stage repeated,
+    // or one more array, turned the order of the two forms round); y stays as it is
+    const double cg[2] = {1e-3, 1e-3};
+    StageUpdate u[4];
+    double2* in[4];
+    rk4_stages(0.0, u, in);
+    u[0].mon = nullptr;
+    auto step = [&](int f) {
+        for (int i = 0; i < 4; ++i) {
+            CommArgs c = tuning_stage_args(kind[f]);
+            c.rho = in[i];
+            c.up = u[i];
+            c.D = c.D2 = nullptr;
+            // with exchange the derivative alone: T and W are not allocated yet, and on
+            // these grids the exchange term's passes are the same in either form
+            if (coulomb)
+                c.D = gradient(c.rho, cg, nullptr, true, true);
+            else
+                derivative_terms(c, cg, nullptr, nullptr, nullptr, true, true);
+            launch_comm(nb, layout, kind[f], tile[f], c, s);
+        }
+    };
+    hipEvent_t e0, e1;
+    HIP_CHECK(hipEventCreate(&e0));
+    HIP_CHECK(hipEventCreate(&e1));
+    float best[2] = {1e30f, 1e30f};
+    for (int trial = 0; trial < 3; ++trial)
+        for (int f = 0; f < 2; ++f) {
+            grad_fused = f == 1;
+            step(f);  // warm-up
+            HIP_CHECK(hipEventRecord(e0, s));
+            for (int r = 0; r < 3; ++r) step(f);
+            HIP_CHECK(hipEventRecord(e1, s));
+            HIP_CHECK(hipEventSynchronize(e1));
+            float ms = 0.f;
+            HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
+            best[f] = std::min(best[f], ms);
+        }
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    HIP_CHECK(hipGetLastError());
+    grad_fused = best[1] < 0.98f * best[0];  // the two passes unless the other form is clearly faster
+    tuned_grad()[gkey] = grad_fused;
 }
 
 // The commutator's operands in the RK4 step's heaviest stage (the third),

@@ -247,6 +247,8 @@ class Engine {
     void fock(const double2* in, bool row_done = false);
     void build_velocity(double det);
     void autotune();
+    void tune_commutator();
+    void tune_gradient();
     CommArgs tuning_stage_args(int kind) const;
     AxisFFTArgs axis_args(int axis, const FFTChoice& c, int mode, const double2* in, const double2* addend,
                           double2* out, double coef, double scale, const double* mult) const;
