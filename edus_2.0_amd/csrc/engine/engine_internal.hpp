@@ -132,15 +132,21 @@ class Engine {
     // bytes as two passes (the second one reads the first one's result) without
     // the second launch and its wait: 45 x 63, 21 planes 4.8 us instead of 10 (plane
     // kernel), 120 x 120, 196 planes 31.8 instead of 41.9.  Line splits with a
-    // factor of 11 or above 12 are taken up to a plane set of 8 MB: on large grids
-    // the second result, one more array in the cache behind HBM, costs the
-    // commutator more than the launch gains (240 x 180, 100 planes: 48.3 us, two
-    // passes 69.5, but ten steps 4099 against 3781).  Like plane_pass, not a function
-    // of the number of stacked instances.
+    // factor of 11 or above 12 (more registers, fewer waves) are taken up to a plane
+    // set of 8 MB, and above that where an axis has no two-step kernel and would take
+    // the Stockham one, unless the plane fits in LDS.  Ten steps in us, otherwise and
+    // in one launch: Stockham passes, 10 bands 112 x 112 (19 MB) 4117, 2044, 14 bands
+    // 112 x 112 (38 MB) 6905, 3370, 14 bands 176 x 168 (88 MB) 17324, 8279; two
+    // two-step passes, 7 bands 128 x 128 (12 MB) 1547, 1531, 14 bands (49 MB) 4343,
+    // 4406, 10 bands 240 x 180 (66 MB) 6129, 6568; plane in LDS, 12 bands 66 x 65
+    // (9 MB) 1397, 1421, 14 bands 77 x 91 (21 MB) 2010, 2288.  Like plane_pass, not a
+    // function of the number of stacked instances.
     bool axes_together() const
     {
-        return !kgrad && !coulomb && !peierls && axes_available(N0, N1) && !(grad_form_choice(N0, N1) && grad_fused) &&
-               (!axes_wide(N0, N1) || size_t(npl) * Nk * sizeof(double2) <= kAxesSmallBytes);
+        if (kgrad || coulomb || peierls || !axes_available(N0, N1) || (grad_form_choice(N0, N1) && grad_fused))
+            return false;
+        const bool stockham = !fft_choice[0].two_step || !fft_choice[1].two_step;
+        return !axes_wide(N0, N1) || size_t(npl) * Nk * sizeof(double2) <= kAxesSmallBytes || (stockham && !plane_ok);
     }
     // k-space gradient: the stencil's taps read by the commutator itself (RK4,
     // whose stages never overwrite their input)
