@@ -87,8 +87,13 @@ struct Tile {
                 if (kk < ke) {
                     // the row of ones lies behind the operand's own rows
                     v[e] = load4<VEC>(X + long(kk) * sk + rr, rr, ones >= 0 ? ones : rows);
-                    const int o = ones - rr;
-                    if (ones >= 0 && o >= 0 && o < 4) reinterpret_cast<uint16_t*>(&v[e])[o] = 0x3f80;
+                    // (an index into v[e] at run time would put it in scratch memory)
+                    if (ones >= 0) {
+                        v[e].x = rr == ones ? 0x3f80 : v[e].x;
+                        v[e].y = rr + 1 == ones ? 0x3f80 : v[e].y;
+                        v[e].z = rr + 2 == ones ? 0x3f80 : v[e].z;
+                        v[e].w = rr + 3 == ones ? 0x3f80 : v[e].w;
+                    }
                 }
             }
         }
