@@ -257,16 +257,20 @@ bool axes_wide(int N0, int N1);  // a factor of 11 or above 12 (more registers)
 PlaneArgs axes_args(int N0, int N1);
 void launch_axes(const PlaneArgs& a, hipStream_t s);
 bool plane_available(int N0, int N1);
-// grids on which the tuning chooses between the one-pass derivative
-// (plane_fft.hip, or grad_fused.hip where the plane does not fit) and axis passes
+// grids on which the tuning chooses between the one-pass derivative and axis
+// passes (edus_set_tuning's grad_fused): those with a kernel in grad_fused.hip, and
+// two whose planes just fill the LDS of a CU.  On others there is nothing to choose:
+// smaller planes are left to the axis passes (plane_fft.hip has the figures), and
+// with a Stockham axis the plane kernel or axes_kernel was the faster one at every
+// size measured.
 inline bool grad_form_choice(int N0, int N1)
 {
-    return N0 == N1 && (N0 == 120 || N0 == 96 || N0 == 90 || N0 == 48);
+    return grad_fused_available(N0, N1) || (N0 == N1 && (N0 == 96 || N0 == 90));
 }
 // of those, the ones whose one-pass derivative is plane_fft.hip's (90 x 90 and
 // 196 planes: 21.1 us, grad_fused.hip took 23.0; 96 x 96: 22.4 and 28.3; at
 // 48 x 48 and 784 planes grad_fused.hip takes 20.1, plane_fft.hip 22.8)
-inline bool plane_form(int N0, int N1) { return N0 == N1 && (N0 == 96 || N0 == 90); }
+inline bool plane_form(int N0, int N1) { return grad_form_choice(N0, N1) && !grad_fused_available(N0, N1); }
 PlaneArgs plane_args(int N0, int N1);  // sizes and line splits
 void launch_plane(const PlaneArgs& a, hipStream_t s);
 void launch_plane_permute(const double* W, double* Wp, int P, int N0, int N1, hipStream_t s);

@@ -222,7 +222,8 @@ int edus_timing_get(edus_ctx* ctx, const char* kernel_class, double* total_ms, l
  *   comm_tile_ab   the same for the Adams-Bashforth steps
  *   grad_fused     1: the spectral derivative in one pass per plane (one
  *                  work-group holds a plane: grids 120 x 120, 96 x 96,
- *                  90 x 90, 48 x 48; on the last three the exchange term too);
+ *                  90 x 90, 48 x 48; on the last three the exchange term too,
+ *                  in the Peierls gauge the phase on 96 x 96 and 90 x 90);
  *                  0: axis passes, both axes' in one launch.  Other grids
  *                  have no choice (0): with exchange planes that fit in LDS go
  *                  one work-group per plane; without, both axes' passes share a
