@@ -11,8 +11,7 @@ namespace edus {
 // While set (by an AttributesOnly guard), the launch functions only raise
 // their kernels' dynamic-LDS limit (hipFuncSetAttribute, once per kernel) and
 // launch nothing.  Engines do this for every kernel they may launch before
-// any hipGraph capture: a limit first raised while a stream is being captured
-// does not reach the captured launch.
+// any hipGraph capture, so that no limit is first raised during one.
 extern thread_local bool g_attributes_only;
 struct AttributesOnly {
     AttributesOnly() { g_attributes_only = true; }

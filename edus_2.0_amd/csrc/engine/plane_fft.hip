@@ -26,9 +26,10 @@
 // Neighbouring lanes take neighbouring lines: columns are adjacent words, and
 // rows are N1 | 1 elements apart, so neither axis has bank conflicts.
 //
-// What bounds it: the FP64 transforms and LDS round trips (12 of 16 B per
-// element for both axes) of one plane on one CU; with fewer planes than CUs the
-// chip is partly idle, which the saved launches and passes outweigh.  Measured
+// What bounds it: a chain of up to seven steps of one plane on one CU, a barrier
+// between each and about one round of tasks in a step (90 x 90 with exchange: the
+// FP64 operations alone would take 4 of its 19 us, its bytes 5); with fewer planes
+// than CUs the chip is partly idle, which the saved launches and passes outweigh.  Measured
 // (derivative): 45 x 63, 21 planes 10 us, two Stockham passes 27; 90 x 90 with
 // exchange, 64 planes 18.9 us, four axis passes 32; 96 x 96, 784 planes 82 us
 // (2.8 TB/s), two axis passes 90.  A derivative alone on a small grid with
@@ -323,7 +324,8 @@ __global__ void __launch_bounds__(NT, MAXR <= 12 ? 4 : 2) plane_kernel(PlaneArgs
 // a launch costs what it computes, this saves the second launch and its wait
 // for the first.  Bound by latency there: three barriers and the launch.  On
 // large ones by memory and the lanes at work (axes_best_shape): 120 x 120, 196
-// planes 31.8 us, 5.7 TB/s of its two reads and two writes.
+// planes 31.8 us by itself and 36.3 in the step, 5.7 and 5.0 TB/s of its two
+// reads and two writes, both reads of the planes from memory.
 template <int MAXR>
 __global__ void __launch_bounds__(kAxesMaxThreads, MAXR <= 12 ? 4 : 3) axes_kernel(PlaneArgs a, int nb0, int L0, int L1)
 {
