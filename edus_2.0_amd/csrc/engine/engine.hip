@@ -832,7 +832,7 @@ void Engine::tune_gradient()
     }
     // an RK4 step of length 0 on the arrays of a real one (at 14 bands on 120 x 120
     // these are about the size of the cache behind HBM, and a single stage repeated,
-    // or one more array, turned the order of the two forms round); y stays as it is
+    // or one more array, turned the order of the two forms round); the state is not set yet
     const double cg[2] = {1e-3, 1e-3};
     StageUpdate u[4];
     double2* in[4];
@@ -872,6 +872,7 @@ void Engine::tune_gradient()
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipMemsetAsync(y, 0, plane_bytes(), s));  // also where H0 holds no numbers
     grad_fused = best[1] < 0.98f * best[0];  // the two passes unless the other form is clearly faster
     tuned_grad()[gkey] = grad_fused;
 }

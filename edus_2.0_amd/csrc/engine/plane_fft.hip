@@ -13,7 +13,7 @@
 // convolution of one plane are two work-groups of the same launch.
 //
 // Every line is n = RA * RB with both factors at most 16, chosen on the host
-// (plane_plan); the factors are run-time values and each step is dispatched on
+// (plane_args); the factors are run-time values and each step is dispatched on
 // its radix, so that every axis length with such a split shares one kernel.
 // Element j = ja RB + jb, frequency k = ka + RA kb:
 //   A   DFT_RA over ja, times w^(jb ka), to position ka RB + jb;

@@ -38,3 +38,12 @@ def test_a_group_keeps_its_members_form(n, nb):
         t.grad_fused = form
         a.set_tuning(t)
         assert a.clone().get_tuning().grad_fused == form
+
+
+@pytest.mark.parametrize("n", [96, 120])
+def test_tuning_leaves_no_state(n):
+    """A context starts from rho = 0, also where H0 holds a NaN."""
+    h = np.zeros((n * n, 2, 2), dtype=complex)
+    h[5, 0, 0] = np.nan
+    eng = edus.Engine(2, n, n, h, A=A, filledbands=1)
+    assert not eng.get_state().any()
